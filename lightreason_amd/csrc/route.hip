@@ -19,7 +19,8 @@
 namespace lrmoe {
 namespace {
 
-constexpr int kTokTile = 16;     // tokens per router workgroup
+constexpr int kTokTile = 16;     // most tokens of a decode call (one tile)
+constexpr int kCus = 256;        // CUs of an MI355X (grid sizing only)
 constexpr int kXStride = kHidden + 8;  // LDS row stride in bf16 (16-byte pad)
 
 // Stage up to 16 token rows of the router input into LDS, applying the
@@ -169,69 +170,217 @@ __device__ int32_t validate_ids(const int32_t* ids, int tokens) {
     return flags;
 }
 
-// Router logits for a tile of <= 16 tokens: 4*RPW router rows per workgroup
-// (RPW rows per wave).  With SHARED_ROW the last blockIdx.y instead computes
-// the shared-expert gate for the tile (wave 0).  PREFILL also clears the
-// bucketing histogram for the top-k kernel that follows on the stream.  No
-// workgroup waits on another: the kernel boundary publishes the logits.
-template <bool PREFILL, int RPW>
+// Router logits of <= 16 tokens: 4 router rows per workgroup, one per wave
+// (the tokens are one tile; the kernel boundary publishes the logits).  With
+// norm, the first workgroup also writes the normalised rows.
 __global__ __launch_bounds__(256) void router_logits(RouteArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t xs[kTokTile * kXStride];
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
-    const int t0 = blockIdx.x * kTokTile;
-    const int count = min(kTokTile, a.tokens - t0);
-    constexpr int kRowGroups = kExperts / (4 * RPW);
-
-    if (PREFILL && blockIdx.x == 0 && blockIdx.y == 0) {
-        if (threadIdx.x == 0) *a.plan.status = 0;
-    }
-
+    const int row = blockIdx.x * 4 + wave;
     // Issue this wave's weight loads before staging the tokens.
-    const bool shared_row = blockIdx.y == kRowGroups;
-    const bool router_rows = !shared_row && a.router != nullptr;
-    const bool gate_row = shared_row && a.shared_gate != nullptr;
-    uint4 wraw[RPW][4];
-    if (router_rows) {
+    uint4 wraw[4];
+    if (a.router != nullptr) {
+        const uint4* src = reinterpret_cast<const uint4*>(a.router + static_cast<size_t>(row) * kHidden + 32 * lane);
 #pragma unroll
-        for (int i = 0; i < RPW; ++i) {
-            const int row = (blockIdx.y * 4 + wave) * RPW + i;
-            const uint4* src = reinterpret_cast<const uint4*>(a.router + static_cast<size_t>(row) * kHidden + 32 * lane);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) wraw[i][q] = src[q];
-        }
-    } else if (gate_row) {
-        const uint4* src = reinterpret_cast<const uint4*>(a.shared_gate + 32 * lane);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) wraw[0][q] = src[q];
+        for (int q = 0; q < 4; ++q) wraw[q] = src[q];
     }
-
-    if (router_rows || gate_row || (blockIdx.y == 0 && a.norm != nullptr)) {
-        stage_tokens(xs, a.x, a.norm, a.eps, t0, count, blockIdx.y == 0 ? a.normed : nullptr);
+    if (a.router != nullptr || (blockIdx.x == 0 && a.norm != nullptr)) {
+        stage_tokens(xs, a.x, a.norm, a.eps, 0, a.tokens, blockIdx.x == 0 ? a.normed : nullptr);
     }
     __syncthreads();
+    if (a.router == nullptr) return;
+    float w[32];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) unpack8(wraw[q], w + 8 * q);
+    for (int t = 0; t < a.tokens; ++t) {
+        const float s = wave_butterfly_sum(lane_dot(w, xs, t, lane));
+        if (lane == 0) a.logits[static_cast<size_t>(t) * kExperts + row] = static_cast<uint16_t>(f2bf(s));
+    }
+}
 
-    if (router_rows) {
+// ---- router of more than 16 tokens --------------------------------------------
+//
+// The canonical sum of a logit is 64 chains of 32 fmaf, met in a balanced
+// binary tree.  v_mfma_f32_16x16x1_4b_f32 runs exactly such chains: with
+// K = 1 every accumulator takes one fused multiply-add per instruction, so 32
+// of them in element order are the chain from +0, for four chains (the
+// instruction's four blocks) of a 16 x 16 tile of (router row, token) at
+// once.  Each wave owns 8 consecutive chains (256 of the 2048 columns) of
+// every tile of its workgroup; their sums, (b0 + b1) + (b2 + b3) per
+// instruction group and then over groups and waves, are the butterfly's tree.
+//
+// Bound by the fp32 matrix rate (this instruction: 129 TFLOP/s measured, fmaf
+// on the VALU 68) and, up to a few hundred tokens, by the latency of one
+// tile.  The VALU form it replaces (one wave per row, a butterfly per dot
+// product) normalised the tokens 17 times and spent ~90 VALU instructions on
+// every 64 x 32 fmaf.  rocprof, T = 40 / 333 / 2048 / 8192 with norm and
+// gate: 23 / 34 / 125 / 438 -> 12 / 21 / 50 / 127 us.
+//
+// Tile: 32 tokens (16 while that gives every tile a CU of its own; their
+// normalised rows stay in registers as B operands) against `per` tiles of 16 router rows; a 17th tile, whose rows all
+// hold the shared-expert gate, gives that gate.  Normalising the tokens
+// costs about 1.5 row tiles; the grid's y dimension trades repeats of it
+// against idle CUs (launch_route).
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr int kRmThreads = 512;
+constexpr int kRmWaves = kRmThreads / kWave;
+constexpr int kRmRowTiles = kExperts / 16;          // router row tiles; tile 16 is the shared gate
+
+__device__ __forceinline__ float bf_elem(const uint4 (&v)[4], int j) {
+    const uint4 p = v[j >> 3];
+    const int w = (j & 7) >> 1;
+    const uint32_t word = w == 0 ? p.x : w == 1 ? p.y : w == 2 ? p.z : p.w;
+    return (j & 1) ? hi_bf(word) : lo_bf(word);
+}
+
+// NT column tiles of 16 tokens per workgroup.
+template <int NT>
+__global__ __launch_bounds__(kRmThreads) void router_tiles(RouteArgs a, int first_tile, int tiles, int per) {
+    constexpr int kTok = 16 * NT;
+    constexpr int kRows = kTok / kRmWaves;  // token rows whose norm scale a wave computes
+    __shared__ __attribute__((aligned(16))) float red[2][kRmWaves][NT][kWave * 4];
+    __shared__ float scale[kTok];
+    const int wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int m = lane & 15;
+    const int t0 = blockIdx.x * kTok;
+    const int tile0 = first_tile + blockIdx.y * per;
+    const int tile1 = min(tile0 + per, first_tile + tiles);
+    // This lane's two pieces of 32 columns (chains 8 wave + lane / 16 and + 4).
+    const int k0 = 32 * (8 * wave + (lane >> 4));
+    uint4 wraw[2][4];
+    auto load_rows = [&](int tile, uint4 (*dst)[4]) {
+        const uint16_t* row = tile < kRmRowTiles ? a.router + static_cast<size_t>(16 * tile + m) * kHidden : a.shared_gate;
 #pragma unroll
-        for (int i = 0; i < RPW; ++i) {
-            const int row = (blockIdx.y * 4 + wave) * RPW + i;
-            float w[32];
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) unpack8(wraw[i][q], w + 8 * q);
-            for (int t = 0; t < count; ++t) {
-                const float s = wave_butterfly_sum(lane_dot(w, xs, t, lane));
-                if (lane == 0) a.logits[static_cast<size_t>(t0 + t) * kExperts + row] = static_cast<uint16_t>(f2bf(s));
+            for (int i = 0; i < 4; ++i) dst[q][i] = ldg16(row + k0 + 128 * q + 8 * i);
+    };
+    // Token rows past the last repeat it; their results are dropped.
+    uint4 x[NT][2][4];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const uint16_t* row = a.x + static_cast<size_t>(min(t0 + 16 * n + m, a.tokens - 1)) * kHidden;
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[n][q][i] = ldg16(row + k0 + 128 * q + 8 * i);
+    }
+    if (a.norm != nullptr) {
+        uint4 rows[kRows][4], nw[2][4];
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            const int t = min(t0 + kRows * wave + i, a.tokens - 1);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) rows[i][q] = ldg16(a.x + static_cast<size_t>(t) * kHidden + 32 * lane + 8 * q);
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) nw[q][i] = ldg16(a.norm + k0 + 128 * q + 8 * i);
+        if (tile0 < tile1) load_rows(tile0, wraw);
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            const float r = row_rms_scale(rows[i], a.eps);
+            if (lane == 0) scale[kRows * wave + i] = r;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const float r = scale[16 * n + m];
+            const int t = t0 + 16 * n + m;
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[n][q][i] = rms_apply8(x[n][q][i], nw[q][i], r);
+            if (blockIdx.y == 0 && t < a.tokens) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        *reinterpret_cast<uint4*>(a.normed + static_cast<size_t>(t) * kHidden + k0 + 128 * q + 8 * i) = x[n][q][i];
             }
         }
-    } else if (gate_row && wave == 0) {
-        float w[32];
+    } else if (tile0 < tile1) {
+        load_rows(tile0, wraw);
+    }
+    // A tile's partial sums meet in LDS; they are added and stored while the
+    // next tile runs (two buffers: a buffer is written again only after the
+    // barrier that follows its reads).
+    auto finish = [&](int tile) {
+        if (threadIdx.x >= NT * 256) return;
+        // Thread -> (column tile n, lane, i): row 4 (lane / 16) + i of column lane % 16.
+        const int n = threadIdx.x >> 8;
+        const int at = threadIdx.x & 255;
+        float p[kRmWaves];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) unpack8(wraw[0][q], w + 8 * q);
-        for (int t = 0; t < count; ++t) {
-            const float z = rbf(wave_butterfly_sum(lane_dot(w, xs, t, lane)));
-            if (lane == 0) a.sg[t0 + t] = static_cast<uint16_t>(f2bf(1.0f / (1.0f + lr_exp(-z))));
+        for (int w = 0; w < kRmWaves; ++w) p[w] = red[(tile - tile0) & 1][w][n][at];
+        const float s = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+        const int t = t0 + 16 * n + ((at >> 2) & 15);
+        const int row = 4 * (at >> 6) + (at & 3);
+        if (t >= a.tokens) return;
+        if (tile < kRmRowTiles) {
+            a.logits[static_cast<size_t>(t) * kExperts + 16 * tile + row] = static_cast<uint16_t>(f2bf(s));
+        } else if (row == 0) {
+            a.sg[t] = static_cast<uint16_t>(f2bf(1.0f / (1.0f + lr_exp(-rbf(s)))));
+        }
+    };
+    for (int tile = tile0; tile < tile1; ++tile) {
+        // The next tile's rows are requested and the previous tile's results
+        // stored ahead of this tile's MFMAs, which cover both.
+        uint4 wnext[2][4];
+        load_rows(min(tile + 1, tile1 - 1), wnext);
+        if (tile > tile0) finish(tile - 1);
+        f32x4 part[NT];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            f32x16 acc[NT];
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[n][i] = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 32; ++j) {
+                const float w = bf_elem(wraw[q], j);
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    acc[n] = __builtin_amdgcn_mfma_f32_16x16x1f32(w, bf_elem(x[n][q], j), acc[n], 0, 0, 0);
+            }
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                f32x4 s;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s[i] = (acc[n][i] + acc[n][4 + i]) + (acc[n][8 + i] + acc[n][12 + i]);
+                part[n] = q == 0 ? s : part[n] + s;
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(&red[(tile - tile0) & 1][wave][n][4 * lane]) = part[n];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wraw[q][i] = wnext[q][i];
+    }
+    if (tile0 < tile1) finish(tile1 - 1);
+}
+
+// Workgroups per token tile: the count whose rounds over the CUs, each
+// costing its row tiles and ~1.5 for the norm, take the least time.
+int router_splits(int token_tiles, int row_tiles) {
+    int best = 1;
+    double best_cost = 1e30;
+    for (int y = 1; y <= row_tiles; ++y) {
+        const int per = (row_tiles + y - 1) / y;
+        const int groups = (row_tiles + per - 1) / per;  // workgroups that have work
+        const double cost = static_cast<double>((token_tiles * groups + kCus - 1) / kCus) * (per + 1.5);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = groups;
         }
     }
+    return best;
 }
 
 // Top-8 of one token by ballot radix selection.  Lane l holds the logits of
@@ -387,14 +536,30 @@ hipError_t launch_route(const RouteArgs& a, hipStream_t stream) {
         // workgroup.
         hipEvent_t start = ev.start;
         if (a.router != nullptr || a.norm != nullptr) {
-            LRMOE_LAUNCH((router_logits<false, 1>), dim3(1, kExperts / 4), dim3(256), 0, stream, start, nullptr, a);
+            LRMOE_LAUNCH(router_logits, dim3(a.router != nullptr ? kExperts / 4 : 1), dim3(256), 0, stream, start, nullptr, a);
             start = nullptr;
         }
         LRMOE_LAUNCH(topk_bucket_small, dim3(1), dim3(1024), 0, stream, start, ev.stop, a);
         return hipGetLastError();
     }
-    const int tiles = (a.tokens + kTokTile - 1) / kTokTile;
-    LRMOE_LAUNCH((router_logits<true, 4>), dim3(tiles, kExperts / 16 + 1), dim3(256), 0, stream, ev.start, nullptr, a);
+    const int row_tiles = (a.router != nullptr ? kRmRowTiles : 0) + (a.shared_gate != nullptr ? 1 : 0);
+    hipEvent_t start = ev.start;
+    if (row_tiles > 0 || a.norm != nullptr) {
+        const int first = a.router != nullptr ? 0 : kRmRowTiles;
+        const int tiles16 = (a.tokens + 15) / 16;
+        if (tiles16 * row_tiles <= kCus) {
+            LRMOE_LAUNCH(router_tiles<1>, dim3(tiles16, row_tiles > 0 ? row_tiles : 1), dim3(kRmThreads), 0, stream,
+                         start, nullptr, a, first, row_tiles, 1);
+        } else {
+            const int tiles32 = (a.tokens + 31) / 32;
+            const int splits = row_tiles > 0 ? router_splits(tiles32, row_tiles) : 1;
+            LRMOE_LAUNCH(router_tiles<2>, dim3(tiles32, splits), dim3(kRmThreads), 0, stream, start, nullptr, a, first,
+                         row_tiles, (row_tiles + splits - 1) / splits);
+        }
+    } else if (start != nullptr) {
+        const hipError_t rec = hipEventRecord(start, stream);
+        if (rec != hipSuccess) return rec;
+    }
     const hipError_t err = launch_prefill_plan(a.logits_in != nullptr ? a.logits_in : a.logits, nullptr, nullptr,
                                                a.indices, a.weights, a.tokens, a.shared_down != nullptr, a.ws, a.plan,
                                                stream);
