@@ -16,16 +16,16 @@
 // lists, gate/up items and then down items:
 //   gate/up   one item per (unit, 128-row tile): 128 gate + 128 up rows
 //             of one expert against up to 128 tokens.  Each of the 8 waves
-//             streams its 32 weight rows (16 gate, 16 up) from HBM straight
-//             into MFMA A operands, two K-chunks ahead; the same waves stage
-//             the unit's token rows in LDS chunk by chunk (three chunks ahead
-//             in registers), shared by all 8 waves, so a weight byte is read
-//             once per 128 tokens and feeds up to 8 16x16x32 MFMAs.  SwiGLU
-//             in the epilogue, act rows out.
+//             streams its 32 weight rows (16 gate, 16 up) from HBM two
+//             K-chunks ahead and passes them through an LDS stage of its own
+//             into MFMA A operands; the same waves stage the unit's token
+//             rows in LDS chunk by chunk, shared by all 8 waves, so a weight
+//             byte is read once per 128 tokens and feeds up to 8 16x16x32
+//             MFMAs.  SwiGLU in the epilogue, act rows out.
 //   down      one item per (unit, 512 output rows): the unit's act rows are
 //             staged in LDS once, then 4 tiles of 128 down rows over k = 512
-//             pass through registers, each wave loading the next tile's rows
-//             while it multiplies the current one; y rows out (bf16).
+//             stream through registers and a wave's LDS stage, two tiles
+//             ahead; y rows out (bf16).
 //   The ordered combine is experts.hip's combine_kernel.
 //
 // A list is a contiguous eighth of the units, served by the workgroups b
@@ -46,14 +46,13 @@ constexpr int kGuTiles = kInner / kGuRows;  // 4 gate/up tiles per expert
 constexpr int kGuChunk = 128;              // k per LDS chunk
 constexpr int kGuChunks = kHidden / kGuChunk;
 constexpr int kGuSteps = kGuChunk / 32;    // MFMA k-steps (and A loads per lane) per chunk
-constexpr int kXsStride = kGuChunk + 8;    // LDS token row stride (bf16)
+constexpr int kXsStride = kGuChunk;        // LDS row stride of token and weight chunks (bf16), swizzled (swz)
 constexpr int kDnThreads = 512;            // down workgroup: 8 waves of 16 output rows
 constexpr int kDnRows = kDnThreads / kWave * 16;  // 128 output rows per down workgroup
 constexpr int kDnTiles = kHidden / kDnRows;       // 16 down tiles per expert
-constexpr int kDnItemTiles = 4;                   // tiles per down item
-constexpr int kDnItems = kDnTiles / kDnItemTiles; // 4 down items per unit
-constexpr int kDnPieces = kPassTok * (kInner / 8) / kDnThreads;  // 16-byte act pieces per thread: a whole unit
-constexpr int kActStride = kInner + 8;     // LDS act row stride (bf16)
+constexpr int kDnItemTiles = 4;                   // tiles per split down item
+constexpr int kDnItems = kDnTiles / kDnItemTiles; // 4 split down items per unit
+constexpr int kDnStage = 2048;                    // bytes of a wave's LDS stage: 16 rows x 64 k
 constexpr uint64_t kPfSpinTicks = 5000000; // 50 ms of the 100 MHz wall clock
 constexpr int32_t kStatusTimeoutPf = LRMOE_STATUS_TIMEOUT;
 
@@ -224,6 +223,18 @@ __device__ __forceinline__ T ld_const(const T* p) {
     return *reinterpret_cast<const __attribute__((address_space(4))) T*>(reinterpret_cast<uintptr_t>(p));
 }
 
+// Weight rows: streamed past the caches where an expert's rows are read once
+// per call, cached where several of its units read them (see
+// launch_prefill_experts).
+template <bool STREAM>
+__device__ __forceinline__ uint4 ld_weight(const uint16_t* p) {
+    return STREAM ? ldg16_nt(p) : ldg16(p);
+}
+
+__device__ __forceinline__ const uint16_t* uniform_ptr(const uint16_t* p) {
+    return reinterpret_cast<const uint16_t*>(uniform64(reinterpret_cast<uintptr_t>(p)));
+}
+
 __device__ __forceinline__ bool load_unit(const ExpertArgs& a, int u, Unit& w) {
     if (u >= ld_const(&a.ws.control->n_units)) return false;
     const int* rec = reinterpret_cast<const int*>(a.ws.units + u);
@@ -249,100 +260,235 @@ __device__ __forceinline__ bool load_unit(const ExpertArgs& a, int u, Unit& w) {
 // gate/up workgroup (128 intermediate rows of one work unit): 8 waves, each
 // owning two 16-row MFMA tiles (tile r = 8 gate rows and the 8 up rows with
 // the same indices).  The waves also move the unit's token rows into LDS,
-// one 128-column chunk at a time.  A wave issues, per chunk, its token pieces
-// three chunks ahead and its weights two chunks ahead, in that order; every
-// wait is then for exactly the data used next (the memory counter retires in
-// order), and two chunks of weights (16 KiB per wave) stay in flight.  With
-// 8 waves per CU each wave has 256 VGPRs for the 3 weight buffers, the 3
-// token-piece buffers and the accumulators.  A B operand read from LDS feeds
-// both row tiles, and the 4 workgroups of a unit each read its token rows
-// once.
+// one 128-column chunk at a time.
+//
+// Weights: a load instruction covers 4 rows x 256 contiguous bytes (lane l:
+// row 4i + l/16, bytes 16(l%16)), non-temporal, and the 16 rows of a tile pass
+// through the wave's own LDS stage into the MFMA layout.  The same bytes
+// requested directly in the MFMA layout (16 rows x 64 bytes per instruction,
+// cached) stream at 5.1 TB/s over 256 workgroups, this way at 6.2-6.4 (a
+// read-only probe over 1.5 GiB).
+//
+// Per chunk a wave issues its token pieces, then its weights, two to three
+// chunks ahead, each into the registers just written to LDS; the waits are
+// then for exactly the data used next (the memory counter retires in order),
+// and two chunks of weights (16 KiB per wave) stay in flight.  A B operand
+// read from LDS feeds both row tiles, and the 4 workgroups of a unit each
+// read its token rows once.
 constexpr int kGuWaves = kGuRows / 16;
 constexpr int kGuThreads = kGuWaves * kWave;
 constexpr int kGuPieces = kPassTok * kGuChunk / 8 / kGuThreads;  // 16-byte token pieces per thread per chunk
-constexpr int kGuWAhead = 2;  // weight chunks in flight ahead of the MFMAs
-constexpr int kGuTAhead = 3;  // token chunks in flight ahead of the MFMAs
+constexpr int kStRows = 32;                                      // both tiles of a wave
+
+// Place of 16-byte piece p of row r in a 256-byte LDS row: ds_read_b128 takes
+// 16 lanes at a time, rows r % 16 of k-group g and the others of g ^ 1, and
+// with the pieces exchanged by r they fall on all 64 banks once (rows padded
+// to 272 bytes spent 40% of the LDS cycles in conflicts).
+__device__ __forceinline__ int swz(int r, int p) { return r * kXsStride + 8 * (p ^ (r & 15)); }
 
 // The K loop for NB 16-token column blocks (blocks past the unit's tokens
-// read rows whose results are dropped), then SwiGLU.  xrow[j] is this
-// thread's token piece j (row xrow_row[j] of the unit, 16 bytes at column
-// 8 * piece of each chunk).
-template <int NB>
-__device__ __forceinline__ void gateup_mfma(const uint16_t* arow0, const uint16_t* arow1, const uint16_t* const* xrow,
-                                            const int* xrow_row, int piece, uint16_t* xs, uint16_t* act0,
-                                            uint16_t* act1, int count) {
+// read rows whose results are dropped), then SwiGLU.  xoff[j]: byte offset in
+// x of this thread's token piece j (unit row tid / 16 + 32 j, 16 bytes at
+// column 8 * (tid % 16) of each chunk).  gate_w / up_w: the wave's first gate
+// and up row (wave-uniform).  LDS addresses are one base per use, a k-step's
+// or load's pieces reached by an xor (4j + g ^ m = (g ^ m) ^ 4j).
+template <int NB, bool STREAM>
+__device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16_t* up_w, const uint16_t* x,
+                                            const uint32_t* xoff, char* xs, char* stage, uint16_t* act0, uint16_t* act1,
+                                            int count) {
     const int lane = threadIdx.x & 63;
     const int m = lane & 15;
     const int g = lane >> 4;
     f32x4 acc[2][NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[0][b] = acc[1][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // Weights of a chunk: kGuSteps k-steps of both tiles, 256 contiguous
-    // bytes per row, so each DRAM row is read in one burst.
-    uint4 wb[kGuWAhead + 1][kGuSteps][2];
-    uint4 xr[kGuTAhead][kGuPieces];
-    auto load_w = [&](int c, uint4 (*dst)[2]) {
+    uint4 wb[2][2][4];  // two chunks in flight: [chunk parity][tile][load]
+    uint4 xr[2][kGuPieces];
+    const uint32_t lane_off = static_cast<uint32_t>(g * kHidden + 8 * m);
+    uint32_t rd = 2 * swz(m, g);                         // operand row m, k-group g
+    uint32_t wr = 2 * swz(g, m);                         // stage row g, piece m
+    const uint32_t st = 2 * swz(threadIdx.x >> 4, m);    // token row tid / 16, piece tid % 16
+    // Each load's first row, kept in scalar registers (with the lane's 32-bit
+    // offset and the chunk as the instruction's immediate).
+    const uint16_t* wrow[2][4];
 #pragma unroll
-        for (int j = 0; j < kGuSteps; ++j) {
-            dst[j][0] = ldg16(arow0 + 32 * (kGuSteps * c + j));
-            dst[j][1] = ldg16(arow1 + 32 * (kGuSteps * c + j));
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            wrow[r][i] = (i < 2 ? gate_w : up_w) + (8 * r + 4 * (i & 1)) * kHidden;
+            asm volatile("" : "+s"(wrow[r][i]));
+        }
+    auto load_w = [&](int c) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wb[c & 1][r][i] = ld_weight<STREAM>(wrow[r][i] + lane_off + c * kGuChunk);
+    };
+    auto stage_w = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            char* dst = stage + (wr ^ (64 * i)) + 1024 * i;
+#pragma unroll
+            for (int r = 0; r < 2; ++r) *reinterpret_cast<uint4*>(dst + 4096 * r) = wb[c & 1][r][i];
         }
     };
-    auto load_t = [&](int c, uint4* dst) {
+    auto load_t = [&](int c) {
 #pragma unroll
-        for (int j = 0; j < kGuPieces; ++j) dst[j] = ldg16(xrow[j] + c * kGuChunk);
+        for (int j = 0; j < kGuPieces; ++j) xr[c & 1][j] = ldg16(reinterpret_cast<const char*>(x) + c * 2 * kGuChunk + xoff[j]);
     };
-    auto store_t = [&](int c, const uint4* src) {
+    auto store_t = [&](int c) {
 #pragma unroll
         for (int j = 0; j < kGuPieces; ++j)
-            *reinterpret_cast<uint4*>(xs + ((c & 1) * kPassTok + xrow_row[j]) * kXsStride + 8 * piece) = src[j];
+            *reinterpret_cast<uint4*>(xs + (c & 1) * kPassTok * 2 * kXsStride + j * 32 * 2 * kXsStride + st) = xr[c & 1][j];
     };
-#pragma unroll
-    for (int c = 0; c < kGuTAhead; ++c) load_t(c, xr[c]);
-#pragma unroll
-    for (int c = 0; c < kGuWAhead; ++c) load_w(c, wb[c]);
-    store_t(0, xr[0]);
-    const uint16_t* xb = xs + m * kXsStride + 8 * g;
+    load_t(0);
+    load_w(0);
+    load_t(1);
+    load_w(1);
+    store_t(0);
+    load_t(2);
+    stage_w(0);
+    load_w(2);
 #pragma unroll
     for (int c = 0; c < kGuChunks; ++c) {
-        // Chunk c is in LDS buffer c & 1; chunk c-1's buffer and registers
-        // are free.
+        asm volatile("" : "+v"(rd), "+v"(wr));  // keeps the xor'd addresses from being held across chunks
+        // Token chunk c is in LDS buffer c & 1; the other buffer is free.
         __syncthreads();
-        if (c + 1 < kGuChunks) store_t(c + 1, xr[(c + 1) % kGuTAhead]);
-        if (c + kGuTAhead < kGuChunks) load_t(c + kGuTAhead, xr[(c + kGuTAhead) % kGuTAhead]);
-        if (c + kGuWAhead < kGuChunks) load_w(c + kGuWAhead, wb[(c + kGuWAhead) % (kGuWAhead + 1)]);
-        const uint16_t* xcb = xb + (c & 1) * kPassTok * kXsStride;
+        if (c + 1 < kGuChunks) store_t(c + 1);
+        if (c + 3 < kGuChunks) load_t(c + 3);
+        const char* xcb = xs + (c & 1) * kPassTok * 2 * kXsStride;
 #pragma unroll
         for (int j = 0; j < kGuSteps; ++j) {
-            const uint4* ab = wb[c % (kGuWAhead + 1)][j];
+            const uint32_t at = rd ^ (64 * j);
+            const uint4 a0 = *reinterpret_cast<const uint4*>(stage + at);
+            const uint4 a1 = *reinterpret_cast<const uint4*>(stage + 4096 + at);
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                const uint4 bv = *reinterpret_cast<const uint4*>(xcb + 16 * b * kXsStride + 32 * j);
-                acc[0][b] = mfma16x16x32(ab[0], bv, acc[0][b]);
-                acc[1][b] = mfma16x16x32(ab[1], bv, acc[1][b]);
+                const uint4 bv = *reinterpret_cast<const uint4*>(xcb + 16 * b * 2 * kXsStride + at);
+                acc[0][b] = mfma16x16x32(a0, bv, acc[0][b]);
+                acc[1][b] = mfma16x16x32(a1, bv, acc[1][b]);
             }
         }
+        __builtin_amdgcn_wave_barrier();
+        if (c + 1 < kGuChunks) stage_w(c + 1);
+        if (c + 3 < kGuChunks) load_w(c + 3);
+        __builtin_amdgcn_wave_barrier();
     }
     // SwiGLU: lanes g < 2 hold gate rows 4g..4g+3 of a tile's 8, lane + 32 the
-    // up rows with the same index.  act0/act1 point at this lane's first act
-    // element of column 0 for tile 0 and 1 (4 consecutive intermediate rows).
+    // up rows with the same index.  One lane-half swap per pair of rows gives
+    // every lane gate and up of two rows (rows 0, 1 in the low half, 2, 3 in
+    // the high half), so all lanes share the activation's arithmetic.
+    // act0/act1 point at this lane's first act element of column 0 for tile 0
+    // and 1 (2 consecutive intermediate rows).
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            f32x4 up;
+            uint32_t v[2];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) up[i] = __shfl_xor(acc[r][b][i], 32, kWave);
-            const int col = 16 * b + m;
-            if (g < 2 && col < count) {
-                uint32_t v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = swiglu_bf16(rbf(acc[r][b][i]), rbf(up[i]));
-                st_agent64((r ? act1 : act0) + static_cast<size_t>(16 * b) * kInner,
-                           static_cast<uint64_t>(v[0] | (v[1] << 16)) | (static_cast<uint64_t>(v[2] | (v[3] << 16)) << 32));
+            for (int i = 0; i < 2; ++i) {
+                const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[r][b][i]), __float_as_uint(acc[r][b][i + 2]),
+                                                                false, false);
+                v[i] = swiglu_bf16(rbf(__uint_as_float(s[0])), rbf(__uint_as_float(s[1])));
             }
+            if (16 * b + m < count) st_agent32((r ? act1 : act0) + static_cast<size_t>(16 * b) * kInner, v[0] | (v[1] << 16));
+            __builtin_amdgcn_sched_barrier(0);  // interleaving more of these costs spills
         }
     }
+}
+
+// A down item: kDnItemTiles (even) tiles of 128 output rows of one unit, NB
+// 16-token column blocks.  (Items of a whole unit while every workgroup gets
+// one, with the act rows staged once instead of four times, took 12-21 us
+// longer at T = 333-2048: the lists end unevenly.)  The unit's act rows are staged in LDS once (rows
+// of 1 KiB, 16-byte piece p of row r at place p ^ r % 16: see swz).  Each wave
+// streams its 16 rows of a tile (16 KiB contiguous) non-temporally, 8 rows x
+// 128 bytes per instruction, two tiles ahead: a piece of 64 k passes from its
+// two registers through the wave's LDS stage into MFMA operands (place p ^ r
+// % 8 of 128-byte rows), and the registers are requested again at once, so
+// the stream never waits for a tile to end.  y rows go out through a buffer
+// whose range ends at the unit's last row (no branch around a store: one would
+// make the compiler wait for every load in flight).  act_bytes, y_bytes: the
+// unit's rows.  Returns the next item, claimed (by thread 0) before the last
+// two tiles, so that no workgroup holds an unstarted item for long.
+template <int NB, bool STREAM>
+__device__ __forceinline__ uint32_t down_item(const uint16_t* act, uint32_t act_bytes, const uint16_t* wrow, uint16_t* y,
+                                              uint32_t y_bytes, char* lds, char* stage, uint32_t* claim) {
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int m = lane & 15;
+    const int g = lane >> 4;
+    uint4 wt[2][16];
+    f32x4 acc[2][NB];
+    const __amdgpu_buffer_rsrc_t yr =
+        __builtin_amdgcn_make_buffer_rsrc(y, 0, static_cast<int>(y_bytes), 0x00020000);
+    // Load q of a piece: rows 8q + lane / 8, bytes 16 (lane % 8) of the piece.
+    const uint32_t lane_off = static_cast<uint32_t>((lane >> 3) * kInner + 8 * (lane & 7));
+    constexpr size_t kTile = static_cast<size_t>(kDnRows) * kInner;
+    auto load_piece = [&](const uint16_t* tile, int set, int p) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) wt[set][2 * p + q] = ld_weight<STREAM>(tile + lane_off + 8 * q * kInner + 64 * p);
+    };
+    {
+        uint4 st[2 * NB];
+#pragma unroll
+        for (int q = 0; q < 2 * NB; ++q) st[q] = ld_agent16(act, static_cast<uint32_t>((tid + kDnThreads * q) * 16), act_bytes);
+#pragma unroll
+        for (int p = 0; p < 8; ++p) load_piece(wrow, 0, p);
+#pragma unroll
+        for (int p = 0; p < 8; ++p) load_piece(wrow + kTile, 1, p);
+        // Piece lane of row tid / 64 + 8q (row % 16 alternates with q).
+#pragma unroll
+        for (int q = 0; q < 2 * NB; ++q) {
+            const int r = (tid >> 6) + 8 * q;
+            *reinterpret_cast<uint4*>(lds + r * 1024 + 16 * (lane ^ (r & 15))) = st[q];
+        }
+    }
+    __syncthreads();
+    uint32_t rd = static_cast<uint32_t>(m * 1024 + 16 * (m ^ g));
+    const uint32_t ws = static_cast<uint32_t>(lane * 16) ^ static_cast<uint32_t>(16 * (lane >> 3));  // row lane / 8, place lane % 8 ^ row
+    const uint32_t rs = static_cast<uint32_t>(m * 128 + 16 * (g ^ (m & 7)));
+    uint32_t yo = static_cast<uint32_t>(m * kHidden + 4 * g) * 2;
+    auto tile_mfma = [&](int set, const uint16_t* ahead) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[0][b] = acc[1][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {
+            __builtin_amdgcn_wave_barrier();
+            if (NB == 8) asm volatile("" : "+v"(rd));
+#pragma unroll
+            for (int q = 0; q < 2; ++q) *reinterpret_cast<uint4*>(stage + ws + 1024 * q) = wt[set][2 * p + q];
+            __builtin_amdgcn_wave_barrier();
+            if (ahead != nullptr) load_piece(ahead, set, p);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const uint4 av = *reinterpret_cast<const uint4*>(stage + (rs ^ (64 * k)));
+                const uint32_t at = (rd ^ (64 * ((2 * p + k) & 3))) + 256 * ((2 * p + k) >> 2);
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    acc[k][b] = mfma16x16x32(av, *reinterpret_cast<const uint4*>(lds + at + 16384 * b), acc[k][b]);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const f32x4 v = acc[0][b] + acc[1][b];
+            typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])}, yr,
+                                                  static_cast<int>(yo + 16 * b * 2 * kHidden), 0, 0);
+        }
+        yo += kDnRows * 2;
+    };
+#pragma unroll 1
+    for (int t = 2; t < kDnItemTiles; t += 2) {
+        wrow += 2 * kTile;
+        tile_mfma(0, wrow);
+        tile_mfma(1, wrow + kTile);
+    }
+    uint32_t claimed = 0u;
+    if (tid == 0) claimed = __builtin_amdgcn_atomic_inc32(claim, 0xffffffffu, __ATOMIC_RELAXED, "agent");
+    tile_mfma(0, nullptr);
+    tile_mfma(1, nullptr);
+    return claimed;
 }
 
 // The expert stage of a prefill layer in one persistent launch: one
@@ -357,6 +503,7 @@ __device__ __forceinline__ void gateup_mfma(const uint16_t* arow0, const uint16_
 // before any down item of its list and a claimed gate/up item never waits,
 // so the waits end whether or not all workgroups are resident.  The claim
 // counters and per-unit counts are zeroed by pf_fill.
+template <bool STREAM>
 __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     __shared__ int claimed_s;
@@ -396,34 +543,32 @@ __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
             const int lane = tid & 63;
             // Token pieces of this thread: piece tid % 16 of unit rows tid / 16 + 32 j
             // (rows past the unit's count repeat its first token).
-            const int piece = tid & 15;
-            const uint16_t* xrow[kGuPieces];
-            int xrow_row[kGuPieces];
+            uint32_t xoff[kGuPieces];
 #pragma unroll
             for (int j = 0; j < kGuPieces; ++j) {
                 const int c = tid / 16 + (kGuThreads / 16) * j;  // token row of the unit, 0..127
                 const int cc = c < w.count ? c : 0;
                 const int t = w.tokens ? w.tokens[cc] : w.pair0 - kTopK * a.tokens + cc;
-                xrow[j] = a.x + static_cast<size_t>(t) * kHidden + 8 * piece;
-                xrow_row[j] = c;
+                xoff[j] = static_cast<uint32_t>(t) * (2 * kHidden) + 16 * (tid & 15);
             }
             const int m = lane & 15;
             const int g = lane >> 4;
             const int nblk = (w.count + 15) / 16;
             // MFMA row m < 8 of tile r is gate row 128*tile + 16*wave + 8r + m, m >= 8
             // the up row with the same index.
-            const uint16_t* rows = m < 8 ? w.gate : w.up;
-            const int row0 = kGuRows * tile + 16 * wave + (m & 7);
-            const uint16_t* arow0 = rows + static_cast<size_t>(row0) * kHidden + 8 * g;
-            const uint16_t* arow1 = rows + static_cast<size_t>(row0 + 8) * kHidden + 8 * g;
-            uint16_t* act0 = a.ws.act + static_cast<size_t>(w.pair0 + m) * kInner + kGuRows * tile + 16 * wave + 4 * g;
+            const size_t row0 = static_cast<size_t>(kGuRows * tile + 16 * __builtin_amdgcn_readfirstlane(wave)) * kHidden;
+            const uint16_t* gate_w = uniform_ptr(w.gate + row0);
+            const uint16_t* up_w = uniform_ptr(w.up + row0);
+            char* xs = reinterpret_cast<char*>(lds);
+            char* stage = xs + 2 * (2 * kPassTok + wave * kStRows) * kXsStride;
+            uint16_t* act0 = a.ws.act + static_cast<size_t>(w.pair0 + m) * kInner + kGuRows * tile + 16 * wave + 4 * (g & 1) + 2 * (g >> 1);
             uint16_t* act1 = act0 + 8;
             if (nblk <= 2) {
-                gateup_mfma<2>(arow0, arow1, xrow, xrow_row, piece, lds, act0, act1, w.count);
+                gateup_mfma<2, STREAM>(gate_w, up_w, a.x, xoff, xs, stage, act0, act1, w.count);
             } else if (nblk <= 4) {
-                gateup_mfma<4>(arow0, arow1, xrow, xrow_row, piece, lds, act0, act1, w.count);
+                gateup_mfma<4, STREAM>(gate_w, up_w, a.x, xoff, xs, stage, act0, act1, w.count);
             } else {
-                gateup_mfma<8>(arow0, arow1, xrow, xrow_row, piece, lds, act0, act1, w.count);
+                gateup_mfma<8, STREAM>(gate_w, up_w, a.x, xoff, xs, stage, act0, act1, w.count);
             }
         }
         __builtin_amdgcn_s_waitcnt(0);  // this wave's act rows are written
@@ -433,66 +578,18 @@ __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
     }
 
     // ---- down items, one per (unit, quarter of the output rows) ----
-    // The unit's act rows are staged in LDS once, then the item's 4 tiles of
-    // 128 rows run in turn.  Each wave holds its 16 rows of a tile over
-    // k = 512 (16 MFMA A operands per lane) in one of two register sets, and
-    // issues the following tile's rows -- after the third tile, the next
-    // item's first -- once the current tile's have arrived, so a wave
-    // always has one tile's rows in flight while it multiplies.  (The
-    // explicit waits keep the memory counter exact around the stores and
-    // branches: it retires in order.)
-    const int wave = tid >> 6;
-    const int lane = tid & 63;
-    const int m = lane & 15;
-    const int g = lane >> 4;
-    struct DnItem {
-        const uint16_t* arow;  // this lane's first weight element of the item's first tile
-        int u, h0, pair0, count;
-    };
-    auto dn_info = [&](int item, DnItem& d) {
-        const int j = item - n_gu;
-        Unit w;
-        d.u = first + j / kDnItems;
-        load_unit(a, d.u, w);
-        d.h0 = kDnRows * kDnItemTiles * (j % kDnItems) + 16 * wave;
-        d.arow = w.down + static_cast<size_t>(d.h0 + m) * kInner + 8 * g;
-        d.pair0 = w.pair0;
-        d.count = w.count;
-    };
-    auto tile_rows = [&](const uint16_t* arow, uint4* wt) {
-#pragma unroll
-        for (int s = 0; s < kInner / 32; ++s) wt[s] = ldg16(arow + 32 * s);
-    };
-    auto tile_mfma = [&](const DnItem& d, int t, const uint4* wt) {
-        const int nb = (d.count + 15) / 16;
-        for (int b = 0; b < nb; ++b) {
-            const uint16_t* bp = lds + (16 * b + m) * kActStride + 8 * g;
-            f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int s = 0; s < kInner / 32; s += 2) {
-                acc0 = mfma16x16x32(wt[s], *reinterpret_cast<const uint4*>(bp + 32 * s), acc0);
-                acc1 = mfma16x16x32(wt[s + 1], *reinterpret_cast<const uint4*>(bp + 32 * (s + 1)), acc1);
-            }
-            const f32x4 y = acc0 + acc1;
-            const int col = 16 * b + m;
-            if (col < d.count) {
-                uint16_t* dst = a.ws.y + static_cast<size_t>(d.pair0 + col) * kHidden + d.h0 + kDnRows * t + 4 * g;
-                *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3]));
-            }
-        }
-    };
-    constexpr size_t kTileStride = static_cast<size_t>(kDnRows) * kInner;
-    uint4 wa[kInner / 32], wb[kInner / 32];
-    DnItem d;
-    if (cur < n_items) {
-        dn_info(cur, d);
-        tile_rows(d.arow, wa);
-    }
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     while (cur < n_items) {
+        uint32_t claimed;
+        const int j = cur - n_gu;
+        const int u = first + j / kDnItems;
+        const int tile0 = kDnItemTiles * (j % kDnItems);
+        Unit w;
+        load_unit(a, u, w);
         // The unit's 4 gate/up items have counted themselves in (bounded wait).
-        if (tid == 0 && ld_agent32(a.ws.unit_done + d.u) < static_cast<uint32_t>(kGuTiles)) {
+        if (tid == 0 && ld_agent32(a.ws.unit_done + u) < static_cast<uint32_t>(kGuTiles)) {
             const uint64_t start = wall_clock64();
-            while (ld_agent32(a.ws.unit_done + d.u) < static_cast<uint32_t>(kGuTiles)) {
+            while (ld_agent32(a.ws.unit_done + u) < static_cast<uint32_t>(kGuTiles)) {
                 if (wall_clock64() - start > kPfSpinTicks) {
                     timeout_s = 1;
                     break;
@@ -500,43 +597,25 @@ __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
                 __builtin_amdgcn_s_sleep(2);
             }
         }
-        __syncthreads();
-        // The unit's act rows (1 KiB each, written by other workgroups of
-        // this launch: agent-scope loads; rows past the unit's count read as
-        // zeros).
-        const uint16_t* act = a.ws.act + static_cast<size_t>(d.pair0) * kInner;
-        const uint32_t act_bytes = static_cast<uint32_t>(d.count) * kInner * 2;
-        uint4 st[kDnPieces];
-#pragma unroll
-        for (int q = 0; q < kDnPieces; ++q) st[q] = ld_agent16(act, static_cast<uint32_t>((tid + kDnThreads * q) * 16), act_bytes);
-#pragma unroll
-        for (int q = 0; q < kDnPieces; ++q) {
-            const int idx = tid + kDnThreads * q;
-            *reinterpret_cast<uint4*>(lds + (idx / 64) * kActStride + 8 * (idx % 64)) = st[q];
+        __syncthreads();  // also: every wave is done with the previous item's act rows
+        const int h0 = kDnRows * tile0 + 16 * wave;
+        const uint16_t* act = a.ws.act + static_cast<size_t>(w.pair0) * kInner;
+        const uint16_t* wrow = uniform_ptr(w.down + static_cast<size_t>(h0) * kInner);
+        uint16_t* y = a.ws.y + static_cast<size_t>(w.pair0) * kHidden + h0;
+        const uint32_t act_bytes = static_cast<uint32_t>(w.count) * kInner * 2;
+        // to the last row's columns of this wave and item
+        const uint32_t y_bytes = static_cast<uint32_t>(w.count) * kHidden * 2 - 2 * h0;
+        char* rows = reinterpret_cast<char*>(lds);
+        char* stage = rows + kPassTok * 1024 + wave * kDnStage;
+        if (w.count <= 32) {
+            claimed = down_item<2, STREAM>(act, act_bytes, wrow, y, y_bytes, rows, stage, claim);
+        } else if (w.count <= 64) {
+            claimed = down_item<4, STREAM>(act, act_bytes, wrow, y, y_bytes, rows, stage, claim);
+        } else {
+            claimed = down_item<8, STREAM>(act, act_bytes, wrow, y, y_bytes, rows, stage, claim);
         }
-        __syncthreads();
-        __builtin_amdgcn_s_waitcnt(0);
-        tile_rows(d.arow + kTileStride, wb);
-        tile_mfma(d, 0, wa);
-        __builtin_amdgcn_s_waitcnt(0);
-        uint32_t claimed = 0u;
-        if (tid == 0) claimed = take();
-        tile_rows(d.arow + 2 * kTileStride, wa);
-        tile_mfma(d, 1, wb);
-        __builtin_amdgcn_s_waitcnt(0);
-        tile_rows(d.arow + 3 * kTileStride, wb);
-        tile_mfma(d, 2, wa);
-        const int next = publish(claimed);
-        DnItem dn = d;  // past the list's end: a harmless reload of this item's first tile
-        if (next < n_items) dn_info(next, dn);
-        __builtin_amdgcn_s_waitcnt(0);
-        tile_rows(dn.arow, wa);
-        tile_mfma(d, 3, wb);
-        __syncthreads();  // every wave is done with the act rows in LDS
-        cur = next;
-        d = dn;
+        cur = publish(claimed);
     }
-    __builtin_amdgcn_s_waitcnt(0);  // the last reload is dropped
     if (tid == 0 && timeout_s) atomicOr(&a.ws.control->status, kStatusTimeoutPf);
 }
 
@@ -547,8 +626,8 @@ int max_units(int tokens) {
 }  // namespace
 
 size_t prefill_experts_lds() {
-    const size_t gateup = static_cast<size_t>(2) * kPassTok * kXsStride * sizeof(uint16_t);
-    const size_t down = static_cast<size_t>(kPassTok) * kActStride * sizeof(uint16_t);
+    const size_t gateup = static_cast<size_t>(2 * kPassTok + kGuWaves * kStRows) * kXsStride * sizeof(uint16_t);
+    const size_t down = static_cast<size_t>(kPassTok) * kInner * sizeof(uint16_t) + kDnThreads / kWave * kDnStage;
     return gateup > down ? gateup : down;
 }
 
@@ -572,9 +651,11 @@ hipError_t launch_prefill_experts(const ExpertArgs& a, hipStream_t stream) {
     if (device < 0 || device >= 64) return hipErrorInvalidDevice;
     static int cus[64] = {0};  // per device: CU count, 0 until the LDS limit is raised
     if (cus[device] == 0) {
-        err = hipFuncSetAttribute(reinterpret_cast<const void*>(pf_experts), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  static_cast<int>(prefill_experts_lds()));
-        if (err != hipSuccess) return err;
+        for (const void* kernel : {reinterpret_cast<const void*>(pf_experts<true>), reinterpret_cast<const void*>(pf_experts<false>)}) {
+            err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      static_cast<int>(prefill_experts_lds()));
+            if (err != hipSuccess) return err;
+        }
         int n = 0;
         err = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device);
         if (err != hipSuccess) return err;
@@ -585,7 +666,16 @@ hipError_t launch_prefill_experts(const ExpertArgs& a, hipStream_t stream) {
     const int grid = cus[device] / 8 * 8;
     if (grid < 8) return hipErrorNotSupported;
     const StageEvents ev = timing_events(kStageGateUp);
-    LRMOE_LAUNCH(pf_experts, dim3(grid), dim3(kDnThreads), prefill_experts_lds(), stream, ev.start, ev.stop, a);
+    // Below kCachedTokens most experts are one unit and their rows are read
+    // once: non-temporal loads.  Above it several units of an expert share its
+    // rows through the caches.  Layer, non-temporal / cached: T = 333 318 /
+    // 354 us, 2048 426 / 438, 2800 505 / 495, 4000 618 / 576, 8192 1054 / 945.
+    constexpr int kCachedTokens = 2560;
+    if (a.tokens < kCachedTokens) {
+        LRMOE_LAUNCH(pf_experts<true>, dim3(grid), dim3(kDnThreads), prefill_experts_lds(), stream, ev.start, ev.stop, a);
+    } else {
+        LRMOE_LAUNCH(pf_experts<false>, dim3(grid), dim3(kDnThreads), prefill_experts_lds(), stream, ev.start, ev.stop, a);
+    }
     return hipGetLastError();
 }
 

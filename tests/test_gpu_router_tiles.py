@@ -39,11 +39,13 @@ def _check(x, router, norm, gate, oracle, eps=1e-6):
     assert ws.status() == 0
 
 
-@pytest.mark.parametrize("tokens", [17, 31, 32, 33, 240, 241, 257, 600, 2080, 4100])
-@pytest.mark.parametrize("norm,gate", [(True, True), (False, True), (True, False), (False, False)])
+FORMS = [(True, True), (False, True), (True, False), (False, False)]
+
+
+@pytest.mark.parametrize("tokens,norm,gate",
+                         [(t, *form) for t in (17, 31, 32, 33, 240, 241, 257) for form in FORMS]
+                         + [(t, True, True) for t in (600, 2080, 4100)])  # the oracle takes seconds there
 def test_router_tiles_bit_exact(model, oracle, tokens, norm, gate):
-    if tokens > 300 and not (norm and gate):
-        pytest.skip("one form at the sizes where the oracle takes seconds")
     layer = model.layers[0]
     print(f"[router] T={tokens} norm={norm} gate={gate}", flush=True)
     _check(model.hidden(tokens, step=7000 + tokens), layer.router, layer.norm_weight if norm else None,
