@@ -127,13 +127,43 @@ __global__ __launch_bounds__(256) void pf_scan(int nblk, Workspace ws, Plan plan
     }
 }
 
+// SCAN: the masks are counted here (see kScanBlocks), else by pf_scan.
+template <bool SCAN>
 __global__ __launch_bounds__(256) void pf_fill(const int64_t* indices, int tokens, int shared_present, Workspace ws,
                                                Plan plan) {
     __shared__ uint32_t scratch[4];
-    __shared__ uint32_t off[kExperts];
+    __shared__ uint32_t start[kExperts];  // the block's first pair of each expert
+    __shared__ int32_t status_s;
     const int blk = blockIdx.x;
     const int e = threadIdx.x;
-    const int32_t status = *plan.status;
+    uint32_t count = 0, before = 0;  // the expert's pairs: all, and those of earlier blocks
+    int32_t status;
+    if constexpr (SCAN) {
+        if (threadIdx.x == 0) status_s = 0;
+        __syncthreads();
+        const uint8_t* row = ws.bmask + static_cast<size_t>(e) * ws.nblk_pad;
+        const int nblk = gridDim.x;
+        const int32_t flags = e < nblk ? ws.bstatus[e] : 0;  // nblk <= kScanBlocks = 256
+#pragma unroll 4
+        for (int b = 0; b < ws.nblk_pad; b += 16) {
+            const uint4 v = ldg16(row + b);
+            const uint32_t word[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                count += __popc(word[i]);
+                const int bytes = min(max(blk - b - 4 * i, 0), 4);  // of the word, in blocks before blk
+                before += __popc(static_cast<uint32_t>(word[i] & ((1ull << (8 * bytes)) - 1ull)));
+            }
+        }
+        if (flags) atomicOr(&status_s, flags);
+        __syncthreads();
+        status = status_s;
+        if (blk == 0 && threadIdx.x == 0) *plan.status = status;
+    } else {
+        status = *plan.status;
+        count = ws.counts[e];
+        before = ws.blk_base[static_cast<size_t>(e) * ws.nblk_pad + blk];
+    }
     if (status != 0) {
         for (int i = threadIdx.x; i < kBlkTok * kTopK; i += 256) {
             const int t = blk * kBlkTok + i / kTopK;
@@ -299,6 +329,10 @@ __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16
     const int lane = threadIdx.x & 63;
     const int m = lane & 15;
     const int g = lane >> 4;
+    // Full units of calls with many tokens per expert: MFMAs and LDS are the
+    // larger part there.  (Where the weight stream bounds the call the second
+    // barrier per chunk only costs: T = 1000-2048 1-3% slower.)
+    constexpr bool kTurns = NB == kPassTok / 16 && !STREAM;
     f32x4 acc[2][NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[0][b] = acc[1][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -341,38 +375,129 @@ __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16
         for (int j = 0; j < kGuPieces; ++j)
             *reinterpret_cast<uint4*>(xs + (c & 1) * kPassTok * 2 * kXsStride + j * 32 * 2 * kXsStride + st) = xr[c & 1][j];
     };
-    load_t(0);
-    load_w(0);
-    load_t(1);
-    load_w(1);
-    store_t(0);
-    load_t(2);
-    stage_w(0);
-    load_w(2);
-#pragma unroll
-    for (int c = 0; c < kGuChunks; ++c) {
-        asm volatile("" : "+v"(rd), "+v"(wr));  // keeps the xor'd addresses from being held across chunks
-        // Token chunk c is in LDS buffer c & 1; the other buffer is free.
-        __syncthreads();
-        if (c + 1 < kGuChunks) store_t(c + 1);
-        if (c + 3 < kGuChunks) load_t(c + 3);
+    auto multiply = [&](int c) {
         const char* xcb = xs + (c & 1) * kPassTok * 2 * kXsStride;
+        if constexpr (kTurns) {
+            // Pinned order: B operands are read kAhead column blocks ahead of
+            // their MFMAs (left to itself the compiler reads two, waits and
+            // multiplies).
+            constexpr int kAhead = 5;
+            uint4 bv[kAhead + 1];
+            uint4 av[2][2];
+            auto read_a = [&](int j) {
 #pragma unroll
-        for (int j = 0; j < kGuSteps; ++j) {
-            const uint32_t at = rd ^ (64 * j);
-            const uint4 a0 = *reinterpret_cast<const uint4*>(stage + at);
-            const uint4 a1 = *reinterpret_cast<const uint4*>(stage + 4096 + at);
+                for (int r = 0; r < 2; ++r) av[j & 1][r] = *reinterpret_cast<const uint4*>(stage + 4096 * r + (rd ^ (64 * j)));
+            };
+            auto read_b = [&](int i) {
+                bv[i % (kAhead + 1)] = *reinterpret_cast<const uint4*>(xcb + 16 * (i % NB) * 2 * kXsStride + (rd ^ (64 * (i / NB))));
+            };
+            __builtin_amdgcn_sched_barrier(0);
+            read_a(0);
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const uint4 bv = *reinterpret_cast<const uint4*>(xcb + 16 * b * 2 * kXsStride + at);
-                acc[0][b] = mfma16x16x32(a0, bv, acc[0][b]);
-                acc[1][b] = mfma16x16x32(a1, bv, acc[1][b]);
+            for (int i = 0; i < kAhead; ++i) read_b(i);
+#pragma unroll
+            for (int i = 0; i < kGuSteps * NB; ++i) {
+                if (i + kAhead < kGuSteps * NB) read_b(i + kAhead);
+                if (i % NB == 0 && i / NB + 1 < kGuSteps) read_a(i / NB + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) acc[r][i % NB] = mfma16x16x32(av[(i / NB) & 1][r], bv[i % (kAhead + 1)], acc[r][i % NB]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < kGuSteps; ++j) {
+                const uint32_t at = rd ^ (64 * j);
+                const uint4 a0 = *reinterpret_cast<const uint4*>(stage + at);
+                const uint4 a1 = *reinterpret_cast<const uint4*>(stage + 4096 + at);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const uint4 bv = *reinterpret_cast<const uint4*>(xcb + 16 * b * 2 * kXsStride + at);
+                    acc[0][b] = mfma16x16x32(a0, bv, acc[0][b]);
+                    acc[1][b] = mfma16x16x32(a1, bv, acc[1][b]);
+                }
             }
         }
-        __builtin_amdgcn_wave_barrier();
-        if (c + 1 < kGuChunks) stage_w(c + 1);
-        if (c + 3 < kGuChunks) load_w(c + 3);
-        __builtin_amdgcn_wave_barrier();
+    };
+    if constexpr (kTurns) {
+        // The two waves of a SIMD take turns.  In half-step 2c waves
+        // 0-3 multiply chunk c while waves 4-7 move data (stage their weight
+        // chunk c, store their rows of token chunk c + 1, request the next
+        // ones), in half-step 2c + 1 the other way round; a barrier ends every
+        // half-step.  With both waves multiplying and then both moving, a chunk
+        // took 4430 cycles, 2700 of them MFMAs (2048 at full rate).  Layer,
+        // T = 4001 / 8192: 524 / 936 -> 512 / 908 us.
+        // waves 4-7, which store token rows one chunk further ahead (a scalar:
+        // the barriers below sit in branches on it)
+        const int late = __builtin_amdgcn_readfirstlane(threadIdx.x >= kGuThreads / 2 ? 1 : 0);
+        auto load_late = [&](int c, int set) {  // token chunk c + late (past the end: the last again, dropped)
+            const int at = min(c + late, kGuChunks - 1) * 2 * kGuChunk;
+#pragma unroll
+            for (int j = 0; j < kGuPieces; ++j) {
+                uint32_t off = xoff[j];
+                asm volatile("" : "+v"(off));  // scalar base + 32-bit offset, not a 64-bit address held per piece
+                xr[set][j] = ldg16(reinterpret_cast<const char*>(x) + at + off);
+            }
+        };
+        auto store_late = [&](int c, int set) {  // into chunk c + late's buffer
+            char* dst = xs + ((c + late) & 1) * kPassTok * 2 * kXsStride;
+#pragma unroll
+            for (int j = 0; j < kGuPieces; ++j) *reinterpret_cast<uint4*>(dst + j * 32 * 2 * kXsStride + st) = xr[set][j];
+        };
+        load_t(0);
+        load_w(0);
+        load_t(1);
+        load_w(1);
+        store_t(0);
+        load_late(2, 0);
+        __syncthreads();
+        if (late) {
+            store_t(1);
+        }
+        load_late(1, 1);
+        if (late) {
+            stage_w(0);
+            __syncthreads();
+        } else {
+            stage_w(0);
+        }
+        load_w(2);
+#pragma unroll
+        for (int c = 0; c < kGuChunks; ++c) {
+            asm volatile("" : "+v"(rd), "+v"(wr));  // keeps the xor'd addresses from being held across chunks
+            multiply(c);
+            if (c + 1 < kGuChunks) {
+                __syncthreads();
+                stage_w(c + 1);
+                if (c + 3 < kGuChunks) load_w(c + 3);
+                store_late(c + 1, (c + 1) & 1);
+                if (c + 3 < kGuChunks) load_late(c + 3, (c + 1) & 1);
+                __syncthreads();
+            }
+        }
+        if (!late) __syncthreads();
+    } else {
+        load_t(0);
+        load_w(0);
+        load_t(1);
+        load_w(1);
+        store_t(0);
+        load_t(2);
+        stage_w(0);
+        load_w(2);
+#pragma unroll
+        for (int c = 0; c < kGuChunks; ++c) {
+            asm volatile("" : "+v"(rd), "+v"(wr));
+            // Token chunk c is in LDS buffer c & 1; the other buffer is free.
+            __syncthreads();
+            if (c + 1 < kGuChunks) store_t(c + 1);
+            if (c + 3 < kGuChunks) load_t(c + 3);
+            multiply(c);
+            __builtin_amdgcn_wave_barrier();
+            if (c + 1 < kGuChunks) stage_w(c + 1);
+            if (c + 3 < kGuChunks) load_w(c + 3);
+            __builtin_amdgcn_wave_barrier();
+        }
     }
     // SwiGLU: lanes g < 2 hold gate rows 4g..4g+3 of a tile's 8, lane + 32 the
     // up rows with the same index.  One lane-half swap per pair of rows gives
