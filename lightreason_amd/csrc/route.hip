@@ -215,7 +215,7 @@ __global__ __launch_bounds__(256) void router_logits(RouteArgs a) {
 // tile.  The VALU form it replaces (one wave per row, a butterfly per dot
 // product) normalised the tokens 17 times and spent ~90 VALU instructions on
 // every 64 x 32 fmaf.  rocprof, T = 40 / 333 / 2048 / 8192 with norm and
-// gate: 23 / 34 / 125 / 438 -> 12 / 21 / 50 / 127 us.
+// gate: 23 / 34 / 125 / 438 -> 12 / 21 / 46 / 117 us.
 //
 // Tile: 32 tokens (16 while that gives every tile a CU of its own; their
 // normalised rows stay in registers as B operands) against `per` tiles of 16 router rows; a 17th tile, whose rows all
@@ -239,7 +239,7 @@ template <int NT>
 __global__ __launch_bounds__(kRmThreads) void router_tiles(RouteArgs a, int first_tile, int tiles, int per) {
     constexpr int kTok = 16 * NT;
     constexpr int kRows = kTok / kRmWaves;  // token rows whose norm scale a wave computes
-    __shared__ __attribute__((aligned(16))) float red[2][kRmWaves][NT][kWave * 4];
+    __shared__ __attribute__((aligned(16))) float red[3][kRmWaves][NT][kWave * 4];
     __shared__ float scale[kTok];
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
@@ -305,9 +305,15 @@ __global__ __launch_bounds__(kRmThreads) void router_tiles(RouteArgs a, int firs
     } else if (tile0 < tile1) {
         load_rows(tile0, wraw);
     }
-    // A tile's partial sums meet in LDS; they are added and stored while the
-    // next tile runs (two buffers: a buffer is written again only after the
-    // barrier that follows its reads).
+    // A tile's partial sums meet in LDS.  With three or more tiles the waves
+    // 4-7 (`late`) run half a tile behind the others, so that the adding,
+    // storing and unpacking between a SIMD's MFMAs of one wave falls under the
+    // other's: tile t's barrier is at its end for waves 0-3 and in its middle
+    // for waves 4-7, and tile t - 1 is complete after it (three buffers).  In
+    // step a tile took 6.4 us, 4.2 of it MFMAs; routing 2048 / 8192 tokens, plan
+    // included, 52.1 / 130.3 -> 48.8 / 120.7 us.  Fewer tiles only gain the
+    // half-tile wait.  A scalar: barriers sit in branches on it.
+    const bool late = __builtin_amdgcn_readfirstlane(per >= 3 && wave >= kRmWaves / 2);
     auto finish = [&](int tile) {
         if (threadIdx.x >= NT * 256) return;
         // Thread -> (column tile n, lane, i): row 4 (lane / 16) + i of column lane % 16.
@@ -315,7 +321,7 @@ __global__ __launch_bounds__(kRmThreads) void router_tiles(RouteArgs a, int firs
         const int at = threadIdx.x & 255;
         float p[kRmWaves];
 #pragma unroll
-        for (int w = 0; w < kRmWaves; ++w) p[w] = red[(tile - tile0) & 1][w][n][at];
+        for (int w = 0; w < kRmWaves; ++w) p[w] = red[(tile - tile0) % 3][w][n][at];
         const float s = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
         const int t = t0 + 16 * n + ((at >> 2) & 15);
         const int row = 4 * (at >> 6) + (at & 3);
@@ -331,7 +337,7 @@ __global__ __launch_bounds__(kRmThreads) void router_tiles(RouteArgs a, int firs
         // stored ahead of this tile's MFMAs, which cover both.
         uint4 wnext[2][4];
         load_rows(min(tile + 1, tile1 - 1), wnext);
-        if (tile > tile0) finish(tile - 1);
+        if (!late && tile > tile0 + 1) finish(tile - 2);
         f32x4 part[NT];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
@@ -354,16 +360,23 @@ __global__ __launch_bounds__(kRmThreads) void router_tiles(RouteArgs a, int firs
                 for (int i = 0; i < 4; ++i) s[i] = (acc[n][i] + acc[n][4 + i]) + (acc[n][8 + i] + acc[n][12 + i]);
                 part[n] = q == 0 ? s : part[n] + s;
             }
+            if (q == 0 && late) {
+                __syncthreads();
+                if (tile > tile0) finish(tile - 1);
+            }
         }
 #pragma unroll
-        for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(&red[(tile - tile0) & 1][wave][n][4 * lane]) = part[n];
-        __syncthreads();
+        for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(&red[(tile - tile0) % 3][wave][n][4 * lane]) = part[n];
+        if (!late) __syncthreads();
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int i = 0; i < 4; ++i) wraw[q][i] = wnext[q][i];
     }
-    if (tile0 < tile1) finish(tile1 - 1);
+    if (tile0 >= tile1) return;
+    if (!late && tile1 - tile0 > 1) finish(tile1 - 2);
+    __syncthreads();  // the late waves' last sums
+    finish(tile1 - 1);
 }
 
 // Workgroups per token tile: the count whose rounds over the CUs, each
