@@ -48,3 +48,31 @@ def test_units_of_known_size(model, oracle, host_experts, tokens, norm):
         rows = np.unique([0, 15, 16, 127, 128, 129, last - 1, min(last, tokens - 1), tokens - 1])
     want, _, _ = oracle_layer_rows(oracle, layer, xb, host_experts, rows=rows, logits_bits=to_u16(logits))
     assert_layer_close(to_u16(out)[rows], want, xb[rows] if norm else None, what=f"units T={tokens}")
+
+
+@pytest.mark.parametrize("tokens", [65, 121, 128, 129, 2041, 2048, 2049, 2100])
+def test_plan_around_the_scan_launch(device, oracle, tokens):
+    """Up to 2048 tokens (256 blocks) the plan's last kernel counts the block
+    masks itself, above that a scan launch does: whole 16-byte words of masks,
+    their remainders, and both sides of the switch, against the oracle; then
+    a bad route in the last block of each."""
+    from helpers import uniform_routes, zipf_routes
+    from lightreason_amd.moe import Workspace, bucket
+
+    idx, _ = (zipf_routes if tokens % 2 else uniform_routes)(tokens, 100 + tokens)
+    ws = Workspace(device, tokens)
+    ws.buffer.fill_(0xA5)  # nothing may be read that the call did not write
+    print(f"[plan] T={tokens}", flush=True)
+    plan = bucket(torch.from_numpy(idx).to(device), ws)
+    torch.cuda.synchronize()
+    ref = oracle.bucket(idx)
+    unique = int(plan["unique"].item())
+    assert int(plan["status"].item()) == 0 and unique == ref["unique"]
+    np.testing.assert_array_equal(plan["expert"][:unique].cpu().numpy(), ref["expert"])
+    np.testing.assert_array_equal(plan["offset"][:unique + 1].cpu().numpy(), ref["offset"])
+    for name in ("pair_token", "pair_slot", "route_pair"):
+        np.testing.assert_array_equal(plan[name].cpu().numpy(), ref[name])
+    idx[-1, 3] = 256
+    plan = bucket(torch.from_numpy(idx).to(device), ws)
+    assert int(plan["status"].item()) == 1 and int(plan["unique"].item()) == 0
+    assert bool((plan["route_pair"] == -1).all())
