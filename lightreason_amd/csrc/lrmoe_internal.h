@@ -79,7 +79,7 @@ struct Control {
     int32_t status;
     int32_t unique;
     int32_t n_units;    // prefill work units of the current plan
-    uint32_t claim[8];  // prefill: items claimed from each of the 8 work lists (zeroed by pf_fill)
+    uint32_t claim[8];  // prefill: items claimed from each work list (at most 8; zeroed by pf_fill)
     uint32_t reserved[52];
 };
 

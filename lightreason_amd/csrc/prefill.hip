@@ -13,7 +13,7 @@
 //             work units (slot, first pair) of at most kPassTok tokens.
 //
 // Experts (cpu_experts.c:54-69 rounding points; the shared expert is slot 0),
-// one persistent launch (pf_experts) whose workgroups take, from 8 work
+// one persistent launch (pf_experts) whose workgroups take, from 4 work
 // lists, gate/up items and then down items:
 //   gate/up   one item per (unit, 128-row tile): 128 gate + 128 up rows
 //             of one expert against up to 128 tokens.  Each of the 8 waves
@@ -29,10 +29,10 @@
 //             ahead; y rows out (bf16).
 //   The ordered combine is experts.hip's combine_kernel.
 //
-// A list is a contiguous eighth of the units, served by the workgroups b
-// with b % 8 = the list (on XCD b % 8): a unit's token and act rows are
-// fetched into one XCD's L2, and an expert's units (consecutive in the
-// plan) run together on one XCD, its weight tiles shared through that L2.
+// A list is a contiguous quarter of the units, served by the workgroups b with
+// b % 4 = the list (on XCDs b % 8, two per list): a unit's token and act rows
+// are fetched into two L2s, and an expert's units (consecutive in the plan)
+// run together on two XCDs, its weight tiles shared through their L2s.
 // Act rows go out and come back with agent-scope stores and loads, so
 // results do not depend on that placement.
 #include "lrmoe_device.h"
@@ -54,6 +54,12 @@ constexpr int kDnTiles = kHidden / kDnRows;       // 16 down tiles per expert
 constexpr int kDnItemTiles = 4;                   // tiles per split down item
 constexpr int kDnItems = kDnTiles / kDnItemTiles; // 4 split down items per unit
 constexpr int kDnStage = 2048;                    // bytes of a wave's LDS stage: 16 rows x 64 k
+// Work lists of the expert launch, each served by 8 / kLists XCDs: fewer share
+// weight and token rows of neighbouring items less often in one L2, more end
+// less evenly.  Layer with 8 / 4 / 2 / 1 lists: T = 40 215 / 204 / 207 / 208
+// us, 333 309 / 303 / 308 / 317, 2048 418 / 420 / 418 / 429, 8192 968 / 963 /
+// 997 / 1029.
+constexpr int kLists = 4;
 constexpr uint64_t kPfSpinTicks = 5000000; // 50 ms of the 100 MHz wall clock
 constexpr int32_t kStatusTimeoutPf = LRMOE_STATUS_TIMEOUT;
 
@@ -627,10 +633,10 @@ __device__ __forceinline__ uint32_t down_item(const uint16_t* act, uint32_t act_
 }
 
 // The expert stage of a prefill layer in one persistent launch: one
-// workgroup per CU.  Workgroup b serves list b % 8 (a contiguous eighth of
-// the units, so a unit's items and an expert's units share an XCD's L2
-// when workgroup b runs on XCD b % 8): first the 4 gate/up items of each of
-// its units, then
+// workgroup per CU.  Workgroup b serves list b % kLists (a contiguous part of
+// the units, so a unit's items and an expert's units share the L2s of the
+// list's XCDs when workgroup b runs on XCD b % 8): first the 4 gate/up items
+// of each of its units, then
 // the 4 down items of each, claimed from the list's counter one item ahead
 // (a gate/up item claims its successor when it starts, a down item during
 // its third tile).  A down item first waits (bounded) until its unit's 4
@@ -644,10 +650,10 @@ __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
     __shared__ int claimed_s;
     __shared__ int timeout_s;
     const int tid = threadIdx.x;
-    const int list = blockIdx.x % 8;
+    const int list = blockIdx.x % kLists;
     const int n_units = ld_const(&a.ws.control->n_units);
-    const int first = n_units * list / 8;  // the list's units: [first, first + units)
-    const int units = n_units * (list + 1) / 8 - first;
+    const int first = n_units * list / kLists;  // the list's units: [first, first + units)
+    const int units = n_units * (list + 1) / kLists - first;
     const int n_gu = kGuTiles * units;
     const int n_items = n_gu + kDnItems * units;
     uint32_t* claim = &a.ws.control->claim[list];
@@ -801,7 +807,7 @@ hipError_t launch_prefill_experts(const ExpertArgs& a, hipStream_t stream) {
         cus[device] = n;
     }
     // one workgroup per CU (all resident: the down items wait for gate/up
-    // items), a multiple of the 8 lists
+    // items), a multiple of the 8 XCDs
     const int grid = cus[device] / 8 * 8;
     if (grid < 8) return hipErrorNotSupported;
     const StageEvents ev = timing_events(kStageGateUp);
