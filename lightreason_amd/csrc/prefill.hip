@@ -325,6 +325,13 @@ constexpr int kGuWaves = kGuRows / 16;
 constexpr int kGuThreads = kGuWaves * kWave;
 constexpr int kGuPieces = kPassTok * kGuChunk / 8 / kGuThreads;  // 16-byte token pieces per thread per chunk
 constexpr int kStRows = 32;                                      // both tiles of a wave
+constexpr int kGuClaimChunk = kGuChunks - 4;                     // the last weights are requested: claim the next item
+
+// The next item of a list.  (An increment-with-wrap: the compiler's atomic
+// optimiser would turn a lane-0 add into a wave-wide one and wait for it.)
+__device__ __forceinline__ uint32_t claim_item(uint32_t* claim) {
+    return __builtin_amdgcn_atomic_inc32(claim, 0xffffffffu, __ATOMIC_RELAXED, "agent");
+}
 
 // Place of 16-byte piece p of row r in a 256-byte LDS row: ds_read_b128 takes
 // 16 lanes at a time, rows r % 16 of k-group g and the others of g ^ 1, and
@@ -338,10 +345,19 @@ __device__ __forceinline__ int swz(int r, int p) { return r * kXsStride + 8 * (p
 // column 8 * (tid % 16) of each chunk).  gate_w / up_w: the wave's first gate
 // and up row (wave-uniform).  LDS addresses are one base per use, a k-step's
 // or load's pieces reached by an xor (4j + g ^ m = (g ^ m) ^ 4j).
+//
+// claimed (thread 0, STREAM): the next item, claimed late in this one.  A
+// list is served by two XCDs whose workgroups do not start at the same time:
+// claimed as an item starts, the second items of the earlier ones were the
+// first items of the others, and a call of about one item per workgroup took
+// two rounds (T = 1000 on 8 experts, 64 units: 133 us, late 100; 512 tokens on
+// 64 experts 139, 109; one XCD per list, claimed at the start, 97 and 109).
+// The other kernel serves calls of more than two rounds and claims as an item
+// starts: in its loop a late claim costs 21 spills (T = 2560-8192 1-2% slower).
 template <int NB, bool STREAM>
 __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16_t* up_w, const uint16_t* x,
                                             const uint32_t* xoff, char* xs, char* stage, uint16_t* act0, uint16_t* act1,
-                                            int count) {
+                                            int count, uint32_t* claim, uint32_t& claimed) {
     const int lane = threadIdx.x & 63;
     const int m = lane & 15;
     const int g = lane >> 4;
@@ -512,6 +528,7 @@ __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16
             __builtin_amdgcn_wave_barrier();
             if (c + 1 < kGuChunks) stage_w(c + 1);
             if (c + 3 < kGuChunks) load_w(c + 3);
+            if (STREAM && c == kGuClaimChunk && threadIdx.x == 0) claimed = claim_item(claim);
             __builtin_amdgcn_wave_barrier();
         }
     }
@@ -626,7 +643,7 @@ __device__ __forceinline__ uint32_t down_item(const uint16_t* act, uint32_t act_
         tile_mfma(1, wrow + kTile);
     }
     uint32_t claimed = 0u;
-    if (tid == 0) claimed = __builtin_amdgcn_atomic_inc32(claim, 0xffffffffu, __ATOMIC_RELAXED, "agent");
+    if (tid == 0) claimed = claim_item(claim);
     tile_mfma(0, nullptr);
     tile_mfma(1, nullptr);
     return claimed;
@@ -636,14 +653,14 @@ __device__ __forceinline__ uint32_t down_item(const uint16_t* act, uint32_t act_
 // workgroup per CU.  Workgroup b serves list b % kLists (a contiguous part of
 // the units, so a unit's items and an expert's units share the L2s of the
 // list's XCDs when workgroup b runs on XCD b % 8): first the 4 gate/up items
-// of each of its units, then
-// the 4 down items of each, claimed from the list's counter one item ahead
-// (a gate/up item claims its successor when it starts, a down item during
-// its third tile).  A down item first waits (bounded) until its unit's 4
-// gate/up items have counted themselves in.  Every gate/up item is claimed
-// before any down item of its list and a claimed gate/up item never waits,
-// so the waits end whether or not all workgroups are resident.  The claim
-// counters and per-unit counts are zeroed by pf_fill.
+// of each of its units, then the 4 down items of each, claimed from the list's
+// counter one item ahead (a gate/up item claims its successor late in its
+// loop, in the cached kernel as it starts; a down item before its last two
+// tiles).  A down item first waits (bounded) until its unit's 4 gate/up items
+// have counted themselves in.  Every gate/up item is claimed before any down
+// item of its list and a claimed gate/up item never waits, so the waits end
+// whether or not all workgroups are resident.  The claim counters and
+// per-unit counts are zeroed by pf_fill.
 template <bool STREAM>
 __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
@@ -657,7 +674,6 @@ __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
     const int n_gu = kGuTiles * units;
     const int n_items = n_gu + kDnItems * units;
     uint32_t* claim = &a.ws.control->claim[list];
-    auto take = [&]() -> uint32_t { return __builtin_amdgcn_atomic_inc32(claim, 0xffffffffu, __ATOMIC_RELAXED, "agent"); };
     // The claimed item, broadcast to the workgroup (item indices are
     // wave-uniform, so the unit lookups are scalar loads).
     auto publish = [&](uint32_t claimed) -> int {
@@ -668,18 +684,18 @@ __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
         return item;
     };
     if (tid == 0) timeout_s = 0;
-    int cur = publish(tid == 0 ? take() : 0u);
+    int cur = publish(tid == 0 ? claim_item(claim) : 0u);
 
     // ---- gate/up items (every one claimed before any down item) ----
     while (cur < n_gu) {
         uint32_t claimed = 0u;
-        if (tid == 0) claimed = take();
+        if (!STREAM && tid == 0) claimed = claim_item(claim);
         const int u = first + cur / kGuTiles;
         const int tile = cur % kGuTiles;
         // The item's code is written out here rather than called as an
         // inlined function: that form spills registers.
         Unit w;
-        if (load_unit(a, u, w)) {
+        if (load_unit(a, u, w)) {  // always: u < n_units
             const int wave = tid >> 6;
             const int lane = tid & 63;
             // Token pieces of this thread: piece tid % 16 of unit rows tid / 16 + 32 j
@@ -705,11 +721,11 @@ __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
             uint16_t* act0 = a.ws.act + static_cast<size_t>(w.pair0 + m) * kInner + kGuRows * tile + 16 * wave + 4 * (g & 1) + 2 * (g >> 1);
             uint16_t* act1 = act0 + 8;
             if (nblk <= 2) {
-                gateup_mfma<2, STREAM>(gate_w, up_w, a.x, xoff, xs, stage, act0, act1, w.count);
+                gateup_mfma<2, STREAM>(gate_w, up_w, a.x, xoff, xs, stage, act0, act1, w.count, claim, claimed);
             } else if (nblk <= 4) {
-                gateup_mfma<4, STREAM>(gate_w, up_w, a.x, xoff, xs, stage, act0, act1, w.count);
+                gateup_mfma<4, STREAM>(gate_w, up_w, a.x, xoff, xs, stage, act0, act1, w.count, claim, claimed);
             } else {
-                gateup_mfma<8, STREAM>(gate_w, up_w, a.x, xoff, xs, stage, act0, act1, w.count);
+                gateup_mfma<8, STREAM>(gate_w, up_w, a.x, xoff, xs, stage, act0, act1, w.count, claim, claimed);
             }
         }
         __builtin_amdgcn_s_waitcnt(0);  // this wave's act rows are written

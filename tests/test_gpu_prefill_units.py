@@ -76,3 +76,48 @@ def test_plan_around_the_scan_launch(device, oracle, tokens):
     plan = bucket(torch.from_numpy(idx).to(device), ws)
     assert int(plan["status"].item()) == 1 and int(plan["unique"].item()) == 0
     assert bool((plan["route_pair"] == -1).all())
+
+
+def test_one_item_per_workgroup_takes_one_round(model):
+    """1000 tokens on 8 experts are 64 units, 256 gate/up items for 256
+    workgroups; 512 tokens are 128 items.  The larger call must not take a
+    second round (measured 1.08 times the smaller call's time; 1.42 when a
+    workgroup claimed its second item before every one had a first).  Six sets
+    of 8 experts in turn, more weights than the caches hold.  A token's row is
+    the same bits in both calls."""
+    from lightreason_amd.moe import Workspace, moe_experts
+
+    small, large, sets = 512, 1000, 6
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes are chosen for 256 workgroups")
+    x = model.hidden(large, step=8800)
+    rng = np.random.default_rng(88)
+    experts = rng.permutation(256)[:8 * sets].reshape(sets, 8)
+    routes = [torch.from_numpy(np.stack([rng.permutation(e) for _ in range(large)]).astype(np.int64)).to(x.device)
+              for e in experts]
+    weights = torch.softmax(torch.from_numpy(rng.normal(size=(large, 8))), dim=1).to(torch.bfloat16).to(x.device)
+    ptrs = model.layers[0].expert_ptrs
+    ws = {t: Workspace(x.device, t) for t in (small, large)}
+
+    def call(tokens, s):
+        return moe_experts(x[:tokens], routes[s][:tokens], weights[:tokens], ptrs, workspace=ws[tokens])
+
+    def time(tokens):
+        start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        for s in range(sets):
+            call(tokens, s)
+        start.record()
+        for i in range(4 * sets):
+            call(tokens, i % sets)
+        stop.record()
+        stop.synchronize()
+        return start.elapsed_time(stop) / (4 * sets) * 1e3
+
+    print("[units] one item per workgroup", flush=True)
+    for s in range(sets):
+        assert torch.equal(call(small, s).view(torch.int16), call(large, s)[:small].view(torch.int16))
+    assert ws[small].status() == 0 and ws[large].status() == 0
+    times = [(time(small), time(large)) for _ in range(7)]
+    best = [min(t) for t in zip(*times)]
+    print(f"[units] {small} tokens {best[0]:.1f} us, {large} tokens {best[1]:.1f} us", flush=True)
+    assert best[1] < 1.25 * best[0], best
