@@ -270,8 +270,7 @@ __device__ __forceinline__ T ld_const(const T* p) {
 }
 
 // Weight rows: streamed past the caches where an expert's rows are read once
-// per call, cached where several of its units read them (see
-// launch_prefill_experts).
+// per call, cached where several of its units read them (see pf_experts).
 template <bool STREAM>
 __device__ __forceinline__ uint4 ld_weight(const uint16_t* p) {
     return STREAM ? ldg16_nt(p) : ldg16(p);
@@ -346,14 +345,14 @@ __device__ __forceinline__ int swz(int r, int p) { return r * kXsStride + 8 * (p
 // and up row (wave-uniform).  LDS addresses are one base per use, a k-step's
 // or load's pieces reached by an xor (4j + g ^ m = (g ^ m) ^ 4j).
 //
-// claimed (thread 0, STREAM): the next item, claimed late in this one.  A
-// list is served by two XCDs whose workgroups do not start at the same time:
-// claimed as an item starts, the second items of the earlier ones were the
-// first items of the others, and a call of about one item per workgroup took
-// two rounds (T = 1000 on 8 experts, 64 units: 133 us, late 100; 512 tokens on
-// 64 experts 139, 109; one XCD per list, claimed at the start, 97 and 109).
-// The other kernel serves calls of more than two rounds and claims as an item
-// starts: in its loop a late claim costs 21 spills (T = 2560-8192 1-2% slower).
+// claimed (thread 0): the next item, claimed late in this one.  A list is
+// served by two XCDs whose workgroups do not start at the same time: claimed
+// as an item starts, the second items of the earlier ones were the first items
+// of the others, and a call of about one item per workgroup took two rounds
+// (T = 1000 on 8 experts, 64 units: 133 us, late 100; 512 tokens on 64 experts
+// 139, 109; one XCD per list, claimed at the start, 97 and 109).  The
+// streaming loop claims in its last chunks; in the cached one that costs 21
+// spills, and the claim's latency falls under the SwiGLU instead.
 template <int NB, bool STREAM>
 __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16_t* up_w, const uint16_t* x,
                                             const uint32_t* xoff, char* xs, char* stage, uint16_t* act0, uint16_t* act1,
@@ -532,6 +531,7 @@ __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16
             __builtin_amdgcn_wave_barrier();
         }
     }
+    if (!STREAM && threadIdx.x == 0) claimed = claim_item(claim);
     // SwiGLU: lanes g < 2 hold gate rows 4g..4g+3 of a tile's 8, lane + 32 the
     // up rows with the same index.  One lane-half swap per pair of rows gives
     // every lane gate and up of two rows (rows 0, 1 in the low half, 2, 3 in
@@ -654,18 +654,14 @@ __device__ __forceinline__ uint32_t down_item(const uint16_t* act, uint32_t act_
 // the units, so a unit's items and an expert's units share the L2s of the
 // list's XCDs when workgroup b runs on XCD b % 8): first the 4 gate/up items
 // of each of its units, then the 4 down items of each, claimed from the list's
-// counter one item ahead (a gate/up item claims its successor late in its
-// loop, in the cached kernel as it starts; a down item before its last two
-// tiles).  A down item first waits (bounded) until its unit's 4 gate/up items
+// counter one item ahead (a gate/up item claims its successor at its loop's
+// end, a down item before its last two tiles).  A down item first waits (bounded) until its unit's 4 gate/up items
 // have counted themselves in.  Every gate/up item is claimed before any down
 // item of its list and a claimed gate/up item never waits, so the waits end
 // whether or not all workgroups are resident.  The claim counters and
 // per-unit counts are zeroed by pf_fill.
 template <bool STREAM>
-__global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
-    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-    __shared__ int claimed_s;
-    __shared__ int timeout_s;
+__device__ __forceinline__ void expert_items(const ExpertArgs& a, uint16_t* lds, int& claimed_s, int& timeout_s) {
     const int tid = threadIdx.x;
     const int list = blockIdx.x % kLists;
     const int n_units = ld_const(&a.ws.control->n_units);
@@ -689,7 +685,6 @@ __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
     // ---- gate/up items (every one claimed before any down item) ----
     while (cur < n_gu) {
         uint32_t claimed = 0u;
-        if (!STREAM && tid == 0) claimed = claim_item(claim);
         const int u = first + cur / kGuTiles;
         const int tile = cur % kGuTiles;
         // The item's code is written out here rather than called as an
@@ -776,6 +771,26 @@ __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
     if (tid == 0 && timeout_s) atomicOr(&a.ws.control->status, kStatusTimeoutPf);
 }
 
+// Weight rows non-temporal while experts are (nearly) one unit each and their
+// rows are read once; cached, with the half-step turns of full units, from 1.2
+// units per expert on, whose later units find the rows in the caches.  The
+// plan has both counts, the host has neither: tokens say little (128 experts
+// of 129 tokens each are 2064 tokens and two units per expert, 192 of 127 are
+// 3048 and one).  Routed experts, cached over non-temporal time: 0.83-0.97
+// from 1.34 units per expert on, at any token count (96 experts of 129 tokens
+// 252 -> 210 us, 32 of 129 109 -> 91); 1.01-1.05 at 1.02-1.15, 1.05-1.11 at 1
+// (192 of 127 tokens 338 -> 308 us non-temporal); at up to 40 units 0.92-1.05.
+__global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+    __shared__ int claimed_s;
+    __shared__ int timeout_s;
+    if (5 * ld_const(&a.ws.control->n_units) > 6 * ld_const(a.plan.unique)) {
+        expert_items<false>(a, lds, claimed_s, timeout_s);
+    } else {
+        expert_items<true>(a, lds, claimed_s, timeout_s);
+    }
+}
+
 int max_units(int tokens) {
     return (tokens + kPassTok - 1) / kPassTok + kExperts + (kTopK * tokens + kPassTok - 1) / kPassTok;
 }
@@ -812,11 +827,9 @@ hipError_t launch_prefill_experts(const ExpertArgs& a, hipStream_t stream) {
     if (device < 0 || device >= 64) return hipErrorInvalidDevice;
     static int cus[64] = {0};  // per device: CU count, 0 until the LDS limit is raised
     if (cus[device] == 0) {
-        for (const void* kernel : {reinterpret_cast<const void*>(pf_experts<true>), reinterpret_cast<const void*>(pf_experts<false>)}) {
-            err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      static_cast<int>(prefill_experts_lds()));
-            if (err != hipSuccess) return err;
-        }
+        err = hipFuncSetAttribute(reinterpret_cast<const void*>(pf_experts), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  static_cast<int>(prefill_experts_lds()));
+        if (err != hipSuccess) return err;
         int n = 0;
         err = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device);
         if (err != hipSuccess) return err;
@@ -827,16 +840,7 @@ hipError_t launch_prefill_experts(const ExpertArgs& a, hipStream_t stream) {
     const int grid = cus[device] / 8 * 8;
     if (grid < 8) return hipErrorNotSupported;
     const StageEvents ev = timing_events(kStageGateUp);
-    // Below kCachedTokens most experts are one unit and their rows are read
-    // once: non-temporal loads.  Above it several units of an expert share its
-    // rows through the caches.  Layer, non-temporal / cached: T = 333 318 /
-    // 354 us, 2048 426 / 438, 2800 505 / 495, 4000 618 / 576, 8192 1054 / 945.
-    constexpr int kCachedTokens = 2560;
-    if (a.tokens < kCachedTokens) {
-        LRMOE_LAUNCH(pf_experts<true>, dim3(grid), dim3(kDnThreads), prefill_experts_lds(), stream, ev.start, ev.stop, a);
-    } else {
-        LRMOE_LAUNCH(pf_experts<false>, dim3(grid), dim3(kDnThreads), prefill_experts_lds(), stream, ev.start, ev.stop, a);
-    }
+    LRMOE_LAUNCH(pf_experts, dim3(grid), dim3(kDnThreads), prefill_experts_lds(), stream, ev.start, ev.stop, a);
     return hipGetLastError();
 }
 

@@ -2,9 +2,9 @@
 
 All tokens go to the same 8 experts, so every unit's size is known: one
 column block, the edges of the 2-, 4- and 8-block variants (32, 64 and 128
-rows of a unit), a second unit of one row, and the sizes around the switch
-from non-temporal to cached weight rows (2560 tokens).  Outputs of a token
-sample (every token up to 130) against the oracle within
+rows of a unit), and a second unit of one row.  Up to 128 tokens an expert is
+one unit and its weight rows are non-temporal, above that they are cached.
+Outputs of a token sample (every token up to 130) against the oracle within
 helpers.assert_layer_close (1e-2, bf16 storage with fp32 accumulation).
 """
 
@@ -78,24 +78,14 @@ def test_plan_around_the_scan_launch(device, oracle, tokens):
     assert bool((plan["route_pair"] == -1).all())
 
 
-def test_one_item_per_workgroup_takes_one_round(model):
-    """1000 tokens on 8 experts are 64 units, 256 gate/up items for 256
-    workgroups; 512 tokens are 128 items.  The larger call must not take a
-    second round (measured 1.08 times the smaller call's time; 1.42 when a
-    workgroup claimed its second item before every one had a first).  Six sets
-    of 8 experts in turn, more weights than the caches hold.  A token's row is
-    the same bits in both calls."""
+def _two_sizes(model, small, large, routes, weights, x, what):
+    """Routed experts of the first ``small`` and of all ``large`` tokens of
+    every set of ``routes``: a token's row is the same bits in both calls.
+    Returns the best us per call of each size, the sets in turn (more weights
+    than the caches hold)."""
     from lightreason_amd.moe import Workspace, moe_experts
 
-    small, large, sets = 512, 1000, 6
-    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
-        pytest.skip("sizes are chosen for 256 workgroups")
-    x = model.hidden(large, step=8800)
-    rng = np.random.default_rng(88)
-    experts = rng.permutation(256)[:8 * sets].reshape(sets, 8)
-    routes = [torch.from_numpy(np.stack([rng.permutation(e) for _ in range(large)]).astype(np.int64)).to(x.device)
-              for e in experts]
-    weights = torch.softmax(torch.from_numpy(rng.normal(size=(large, 8))), dim=1).to(torch.bfloat16).to(x.device)
+    sets = len(routes)
     ptrs = model.layers[0].expert_ptrs
     ws = {t: Workspace(x.device, t) for t in (small, large)}
 
@@ -113,11 +103,42 @@ def test_one_item_per_workgroup_takes_one_round(model):
         stop.synchronize()
         return start.elapsed_time(stop) / (4 * sets) * 1e3
 
-    print("[units] one item per workgroup", flush=True)
+    print(f"[units] {what}", flush=True)
     for s in range(sets):
         assert torch.equal(call(small, s).view(torch.int16), call(large, s)[:small].view(torch.int16))
     assert ws[small].status() == 0 and ws[large].status() == 0
     times = [(time(small), time(large)) for _ in range(7)]
     best = [min(t) for t in zip(*times)]
     print(f"[units] {small} tokens {best[0]:.1f} us, {large} tokens {best[1]:.1f} us", flush=True)
+    return best
+
+
+def test_one_item_per_workgroup_takes_one_round(model):
+    """1000 tokens on 8 experts are 64 units, 256 gate/up items for 256
+    workgroups; 512 tokens are 128 items.  The larger call must not take a
+    second round (measured 1.08 times the smaller call's time; 1.42 when a
+    workgroup claimed its second item before every one had a first)."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes are chosen for 256 workgroups")
+    rng = np.random.default_rng(88)
+    x = model.hidden(1000, step=8800)
+    experts = rng.permutation(256)[:48].reshape(6, 8)
+    routes = [torch.from_numpy(np.stack([rng.permutation(e) for _ in range(1000)]).astype(np.int64)).to(x.device)
+              for e in experts]
+    weights = torch.softmax(torch.from_numpy(rng.normal(size=(1000, 8))), dim=1).to(torch.bfloat16).to(x.device)
+    best = _two_sizes(model, 512, 1000, routes, weights, x, "one item per workgroup")
     assert best[1] < 1.25 * best[0], best
+
+
+def test_second_units_find_their_rows_cached(model):
+    """96 experts of 128 tokens are one unit each, of 129 two: twice the
+    weight rows read, the second time through the caches (measured 1.24 times
+    the smaller call's time; 1.48 with all rows non-temporal).  The two calls
+    fall on the two sides of the rule that chooses."""
+    rng = np.random.default_rng(96)
+    x = model.hidden(12 * 129, step=8900)
+    token = 8 * np.arange(12 * 129)[:, None] + np.arange(8)[None]  # expert e: tokens e/8, e/8 + 12, ..
+    routes = [torch.from_numpy(rng.permutation(256)[:96][token % 96].astype(np.int64)).to(x.device) for _ in range(2)]
+    weights = torch.softmax(torch.from_numpy(rng.normal(size=(12 * 129, 8))), dim=1).to(torch.bfloat16).to(x.device)
+    best = _two_sizes(model, 12 * 128, 12 * 129, routes, weights, x, "second units")
+    assert best[1] < 1.36 * best[0], best
