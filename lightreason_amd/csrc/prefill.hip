@@ -484,9 +484,7 @@ __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16
         __syncthreads();
         if (late) {
             store_t(1);
-        }
-        load_late(1, 1);
-        if (late) {
+            load_late(1, 1);  // waves 0-3 hold their chunk 1 already
             stage_w(0);
             __syncthreads();
         } else {
