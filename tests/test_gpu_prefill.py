@@ -151,6 +151,16 @@ def test_prefill_t300_router_with_norm(model, oracle, host_experts):
     assert_layer_close(to_u16(out), want, xb, what="T=300 router norm")
 
 
+def test_prefill_t2600_skewed_router(model, oracle, host_experts):
+    """The router on rows with a common direction, in a long prompt: a few
+    experts of several units, most of one unit of every size."""
+    tokens = 2600
+    x = model.hidden(tokens, step=4003).float()
+    direction = model.hidden(1, step=4004).float()
+    x = (x + 0.25 * direction).to(torch.bfloat16)
+    _check(model, oracle, host_experts, x, None, norm=True, what="T=2600 skewed router")
+
+
 def _bf16_bits(values: np.ndarray) -> np.ndarray:
     f32 = np.ascontiguousarray(values, dtype=np.float32)
     bits = f32.view(np.uint32).astype(np.uint64)

@@ -2,8 +2,9 @@
 
 All tokens go to the same 8 experts, so every unit's size is known: one
 column block, the edges of the 2-, 4- and 8-block variants (32, 64 and 128
-rows of a unit), and a second unit of one row.  Up to 128 tokens an expert is
-one unit and its weight rows are non-temporal, above that they are cached.
+rows of a unit).  Up to 128 tokens an expert is one unit and its weight rows
+are non-temporal, above that they are cached: 129-256 tokens are a full unit and
+one at the same edges.
 Outputs of a token sample (every token up to 130) against the oracle within
 helpers.assert_layer_close (1e-2, bf16 storage with fp32 accumulation).
 """
@@ -21,7 +22,8 @@ pytestmark = pytest.mark.gpu
 HOT = np.array([0, 31, 64, 127, 128, 200, 254, 255])
 
 
-@pytest.mark.parametrize("tokens", [17, 32, 33, 48, 49, 64, 65, 127, 128, 129, 2559, 2561])
+@pytest.mark.parametrize("tokens", [17, 32, 33, 48, 49, 64, 65, 127, 128, 129, 159, 160, 161, 192, 193,
+                                    255, 256, 257, 2559, 2561])
 @pytest.mark.parametrize("norm", [False, True])
 def test_units_of_known_size(model, oracle, host_experts, tokens, norm):
     from lightreason_amd.moe import LayerWeights, Workspace, moe_layer
