@@ -13,7 +13,7 @@
 //             work units (slot, first pair) of at most kPassTok tokens.
 //
 // Experts (cpu_experts.c:54-69 rounding points; the shared expert is slot 0),
-// one persistent launch (pf_experts) whose workgroups take, from 4 work
+// one persistent launch (pf_experts) whose workgroups take, from 4 or 8 work
 // lists, gate/up items and then down items:
 //   gate/up   one item per (unit, 128-row tile): 128 gate + 128 up rows
 //             of one expert against up to 128 tokens.  Each of the 8 waves
@@ -29,10 +29,10 @@
 //             ahead; y rows out (bf16).
 //   The ordered combine is experts.hip's combine_kernel.
 //
-// A list is a contiguous quarter of the units, served by the workgroups b with
-// b % 4 = the list (on XCDs b % 8, two per list): a unit's token and act rows
-// are fetched into two L2s, and an expert's units (consecutive in the plan)
-// run together on two XCDs, its weight tiles shared through their L2s.
+// A list is a contiguous part of the units, served by the workgroups b with
+// b % lists = the list (on XCDs b % 8, one or two per list): a unit's token and
+// act rows are fetched into the L2s of its list, and an expert's units
+// (consecutive in the plan) run together there, its weight tiles shared.
 // Act rows go out and come back with agent-scope stores and loads, so
 // results do not depend on that placement.
 #include "lrmoe_device.h"
@@ -54,12 +54,15 @@ constexpr int kDnTiles = kHidden / kDnRows;       // 16 down tiles per expert
 constexpr int kDnItemTiles = 4;                   // tiles per split down item
 constexpr int kDnItems = kDnTiles / kDnItemTiles; // 4 split down items per unit
 constexpr int kDnStage = 2048;                    // bytes of a wave's LDS stage: 16 rows x 64 k
-// Work lists of the expert launch, each served by 8 / kLists XCDs: fewer share
+// Work lists of the expert launch, each served by 8 / lists XCDs: fewer share
 // weight and token rows of neighbouring items less often in one L2, more end
-// less evenly.  Layer with 8 / 4 / 2 / 1 lists: T = 40 215 / 204 / 207 / 208
-// us, 333 309 / 303 / 308 / 317, 2048 418 / 420 / 418 / 429, 8192 968 / 963 /
-// 997 / 1029.
-constexpr int kLists = 4;
+// less evenly.  Rows read once (non-temporal): 8 lists take 1.02-1.06 times as
+// long as 4 up to 512 tokens of a routed prompt and 0.99-1.01 above, 2 lists
+// 1.00-1.03.  Rows that an expert's units share (cached): 8 lists 0.95-0.99 of
+// 4 (T = 5000-8192 0.98, two units on each of 160 experts 0.95-0.97, 24 experts
+// of 257 tokens 0.88), 2 lists 1.02-1.05.
+template <bool STREAM>
+constexpr int kLists = STREAM ? 4 : 8;
 constexpr uint64_t kPfSpinTicks = 5000000; // 50 ms of the 100 MHz wall clock
 constexpr int32_t kStatusTimeoutPf = LRMOE_STATUS_TIMEOUT;
 
@@ -345,13 +348,12 @@ __device__ __forceinline__ int swz(int r, int p) { return r * kXsStride + 8 * (p
 // and up row (wave-uniform).  LDS addresses are one base per use, a k-step's
 // or load's pieces reached by an xor (4j + g ^ m = (g ^ m) ^ 4j).
 //
-// claimed (thread 0): the next item, claimed late in this one.  A list is
-// served by two XCDs whose workgroups do not start at the same time: claimed
+// claimed (thread 0): the next item, claimed late in this one.  A list's
+// workgroups, on two XCDs above all, do not start at the same time: claimed
 // as an item starts, the second items of the earlier ones were the first items
 // of the others, and a call of about one item per workgroup took two rounds
-// (T = 1000 on 8 experts, 64 units: 133 us, late 100; 512 tokens on 64 experts
-// 139, 109; one XCD per list, claimed at the start, 97 and 109).  The
-// streaming loop claims in its last chunks; in the cached one that costs 21
+// (512 tokens on 64 experts, 64 units: 139 us, late 109; one XCD per list,
+// claimed at the start, 109).  The streaming loop claims in its last chunks; in the cached one that costs 21
 // spills, and the claim's latency falls under the SwiGLU instead.
 template <int NB, bool STREAM>
 __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16_t* up_w, const uint16_t* x,
@@ -648,7 +650,7 @@ __device__ __forceinline__ uint32_t down_item(const uint16_t* act, uint32_t act_
 }
 
 // The expert stage of a prefill layer in one persistent launch: one
-// workgroup per CU.  Workgroup b serves list b % kLists (a contiguous part of
+// workgroup per CU.  Workgroup b serves list b % lists (a contiguous part of
 // the units, so a unit's items and an expert's units share the L2s of the
 // list's XCDs when workgroup b runs on XCD b % 8): first the 4 gate/up items
 // of each of its units, then the 4 down items of each, claimed from the list's
@@ -661,10 +663,11 @@ __device__ __forceinline__ uint32_t down_item(const uint16_t* act, uint32_t act_
 template <bool STREAM>
 __device__ __forceinline__ void expert_items(const ExpertArgs& a, uint16_t* lds, int& claimed_s, int& timeout_s) {
     const int tid = threadIdx.x;
-    const int list = blockIdx.x % kLists;
+    constexpr int lists = kLists<STREAM>;
+    const int list = blockIdx.x % lists;
     const int n_units = ld_const(&a.ws.control->n_units);
-    const int first = n_units * list / kLists;  // the list's units: [first, first + units)
-    const int units = n_units * (list + 1) / kLists - first;
+    const int first = n_units * list / lists;  // the list's units: [first, first + units)
+    const int units = n_units * (list + 1) / lists - first;
     const int n_gu = kGuTiles * units;
     const int n_items = n_gu + kDnItems * units;
     uint32_t* claim = &a.ws.control->claim[list];
@@ -776,7 +779,7 @@ __device__ __forceinline__ void expert_items(const ExpertArgs& a, uint16_t* lds,
 // of 129 tokens each are 2064 tokens and two units per expert, 192 of 127 are
 // 3048 and one).  Routed experts, cached over non-temporal time: 0.83-0.97
 // from 1.34 units per expert on, at any token count (96 experts of 129 tokens
-// 252 -> 210 us, 32 of 129 109 -> 91); 1.01-1.05 at 1.02-1.15, 1.05-1.11 at 1
+// 252 -> 205 us, 32 of 129 109 -> 91); 1.01-1.05 at 1.02-1.15, 1.05-1.11 at 1
 // (192 of 127 tokens 338 -> 308 us non-temporal); at up to 40 units 0.92-1.05.
 __global__ __launch_bounds__(kDnThreads, 1) void pf_experts(ExpertArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];

@@ -4,7 +4,7 @@ MI355X).
 
 The prefill plan cuts each expert's token list into work units of at most
 128 tokens (the shared expert's units are tokens 128u .. 128u+127); the
-expert launch gives each of 4 work lists a contiguous range of units.  A
+expert launch gives each of 4 or 8 work lists a contiguous range of units.  A
 unit of more than 64 tokens runs the 8-column-block gate/up MFMA loop and
 stages more than 64 act rows per down item; an expert with more than 128
 tokens is split over several units, which then share a list.  These tests
@@ -171,7 +171,7 @@ def _bf16_bits(values: np.ndarray) -> np.ndarray:
 def test_prefill_concentrated_routes(model, oracle, host_experts, tokens):
     """Every token routed to the same 8 experts (distinct weights per token):
     at T=260 each of them has 3 work units (128, 128, 4 tokens) and the
-    shared expert 3, at T=20 one each -- 27 and 9 units over the 4 lists.
+    shared expert 3, at T=20 one each -- 27 and 9 units over the 8 and 4 lists.
     Every token checked."""
     hot = np.array([3, 40, 77, 100, 150, 201, 230, 255])
     rng = np.random.default_rng(tokens + 11)

@@ -144,3 +144,20 @@ def test_second_units_find_their_rows_cached(model):
     weights = torch.softmax(torch.from_numpy(rng.normal(size=(12 * 129, 8))), dim=1).to(torch.bfloat16).to(x.device)
     best = _two_sizes(model, 12 * 128, 12 * 129, routes, weights, x, "second units")
     assert best[1] < 1.36 * best[0], best
+
+
+def test_lists_of_one_xcd_share_cached_rows(model):
+    """24 experts of 256 tokens are two units each, of 257 three: 288 gate/up
+    items for 256 workgroups, the third units of one row (measured 1.07 times
+    the smaller call's time; 1.20 with lists over two XCDs, whose L2s each
+    fetched an expert's rows)."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes are chosen for 256 workgroups")
+    rng = np.random.default_rng(24)
+    x = model.hidden(3 * 257, step=9000)
+    token = 8 * np.arange(3 * 257)[:, None] + np.arange(8)[None]
+    experts = rng.permutation(256)[:240].reshape(10, 24)
+    routes = [torch.from_numpy(e[token % 24].astype(np.int64)).to(x.device) for e in experts]
+    weights = torch.softmax(torch.from_numpy(rng.normal(size=(3 * 257, 8))), dim=1).to(torch.bfloat16).to(x.device)
+    best = _two_sizes(model, 3 * 256, 3 * 257, routes, weights, x, "lists of one XCD")
+    assert best[1] < 1.14 * best[0], best
