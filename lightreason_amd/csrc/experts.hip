@@ -21,9 +21,9 @@ __device__ __forceinline__ uint4 zero4() { return make_uint4(0, 0, 0, 0); }
 // Ordered combine: one workgroup per token, 8 columns per thread.  Every row
 // is requested as soon as the token's pairs are known, with the slot and
 // weight lookups in their shadow: three round trips in all, where one route
-// after another, each behind its own dependent loads, took 8.8 us at 40 tokens
-// (layer 217 -> 210 us; at 8192 tokens the rows themselves take the time, 68
-// us or 5.3 TB/s, both ways).  Bad routes have pairs of -1: row 0 is read
+// after another, each behind its own dependent loads, took 8.8 us at 40 tokens,
+// this 4.9 (at 8192 tokens the rows themselves take the time, 68 us or 5.3
+// TB/s, both ways).  Bad routes have pairs of -1: row 0 is read
 // then, and dropped.
 __global__ __launch_bounds__(256) void combine_kernel(ExpertArgs a) {
     const int t = blockIdx.x;

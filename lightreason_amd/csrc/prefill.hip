@@ -364,7 +364,7 @@ __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16
     const int g = lane >> 4;
     // Full units of calls with many tokens per expert: MFMAs and LDS are the
     // larger part there.  (Where the weight stream bounds the call the second
-    // barrier per chunk only costs: T = 1000-2048 1-3% slower.)
+    // barrier per chunk only costs: routed prompts of 1000-2048 tokens 1-3%.)
     constexpr bool kTurns = NB == kPassTok / 16 && !STREAM;
     f32x4 acc[2][NB];
 #pragma unroll
@@ -458,8 +458,9 @@ __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16
         // chunk c, store their rows of token chunk c + 1, request the next
         // ones), in half-step 2c + 1 the other way round; a barrier ends every
         // half-step.  With both waves multiplying and then both moving, a chunk
-        // took 4430 cycles, 2700 of them MFMAs (2048 at full rate).  Layer,
-        // T = 4001 / 8192: 524 / 936 -> 512 / 908 us.
+        // took 4430 cycles, 2700 of them MFMAs (2048 at full rate), and the
+        // layer 1.02-1.03 times as long at T = 4001-16384 (16 experts of
+        // 129-384 tokens 1.02-1.06 times).
         // waves 4-7, which store token rows one chunk further ahead (a scalar:
         // the barriers below sit in branches on it)
         const int late = __builtin_amdgcn_readfirstlane(threadIdx.x >= kGuThreads / 2 ? 1 : 0);
@@ -558,12 +559,12 @@ __device__ __forceinline__ void gateup_mfma(const uint16_t* gate_w, const uint16
 // A down item: kDnItemTiles (even) tiles of 128 output rows of one unit, NB
 // 16-token column blocks.  (Items of a whole unit while every workgroup gets
 // one, with the act rows staged once instead of four times, took 12-21 us
-// longer at T = 333-2048: the lists end unevenly.)  The unit's act rows are staged in LDS once (rows
-// of 1 KiB, 16-byte piece p of row r at place p ^ r % 16: see swz).  Each wave
-// streams its 16 rows of a tile (16 KiB contiguous) non-temporally, 8 rows x
-// 128 bytes per instruction, two tiles ahead: a piece of 64 k passes from its
-// two registers through the wave's LDS stage into MFMA operands (place p ^ r
-// % 8 of 128-byte rows), and the registers are requested again at once, so
+// longer at T = 333-2048: the lists end unevenly.)  The unit's act rows are
+// staged in LDS once (rows of 1 KiB, 16-byte piece p of row r at place p ^ r %
+// 16: see swz).  Each wave streams its 16 rows of a tile (16 KiB contiguous), 8
+// rows x 128 bytes per instruction, two tiles ahead: a piece of 64 k passes from
+// its two registers through the wave's LDS stage into MFMA operands (place p ^
+// r % 8 of 128-byte rows), and the registers are requested again at once, so
 // the stream never waits for a tile to end.  y rows go out through a buffer
 // whose range ends at the unit's last row (no branch around a store: one would
 // make the compiler wait for every load in flight).  act_bytes, y_bytes: the

@@ -214,14 +214,14 @@ __global__ __launch_bounds__(256) void router_logits(RouteArgs a) {
 // on the VALU 68) and, up to a few hundred tokens, by the latency of one
 // tile.  The VALU form it replaces (one wave per row, a butterfly per dot
 // product) normalised the tokens 17 times and spent ~90 VALU instructions on
-// every 64 x 32 fmaf.  rocprof, T = 40 / 333 / 2048 / 8192 with norm and
-// gate: 23 / 34 / 125 / 438 -> 12 / 21 / 46 / 117 us.
+// every 64 x 32 fmaf.  rocprof, averages, T = 40 / 333 / 2048 / 8192 with norm
+// and gate: 23 / 34 / 125 / 438 -> 13 / 23 / 48 / 124 us.
 //
 // Tile: 32 tokens (16 while that gives every tile a CU of its own; their
-// normalised rows stay in registers as B operands) against `per` tiles of 16 router rows; a 17th tile, whose rows all
-// hold the shared-expert gate, gives that gate.  Normalising the tokens
-// costs about 1.5 row tiles; the grid's y dimension trades repeats of it
-// against idle CUs (launch_route).
+// normalised rows stay in registers as B operands) against `per` tiles of 16
+// router rows; a 17th tile, whose rows all hold the shared-expert gate, gives
+// that gate.  Normalising the tokens costs about 1.5 row tiles; the grid's y
+// dimension trades repeats of it against idle CUs (launch_route).
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kRmThreads = 512;
 constexpr int kRmWaves = kRmThreads / kWave;
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(kRmThreads) void router_tiles(RouteArgs a, int firs
     // other's: tile t's barrier is at its end for waves 0-3 and in its middle
     // for waves 4-7, and tile t - 1 is complete after it (three buffers).  In
     // step a tile took 6.4 us, 4.2 of it MFMAs; routing 2048 / 8192 tokens, plan
-    // included, 52.1 / 130.3 -> 48.8 / 120.7 us.  Fewer tiles only gain the
+    // included, took 1.07 / 1.08 times as long.  Fewer tiles only gain the
     // half-tile wait.  A scalar: barriers sit in branches on it.
     const bool late = __builtin_amdgcn_readfirstlane(per >= 3 && wave >= kRmWaves / 2);
     auto finish = [&](int tile) {
