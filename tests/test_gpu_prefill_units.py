@@ -161,3 +161,39 @@ def test_lists_of_one_xcd_share_cached_rows(model):
     weights = torch.softmax(torch.from_numpy(rng.normal(size=(3 * 257, 8))), dim=1).to(torch.bfloat16).to(x.device)
     best = _two_sizes(model, 3 * 256, 3 * 257, routes, weights, x, "lists of one XCD")
     assert best[1] < 1.14 * best[0], best
+
+
+def test_captured_call_chooses_at_each_replay(model):
+    """The form of the expert kernel is chosen from the plan on the device: a
+    captured call replays routes on either side of the rule, and bad ones,
+    as an eager call answers them."""
+    from lightreason_amd.moe import Workspace, moe_experts
+
+    tokens = 200
+    rng = np.random.default_rng(200)
+    x = model.hidden(tokens, step=9100)
+    device = x.device
+    few = np.stack([rng.permutation(HOT) for _ in range(tokens)])  # two units per expert: cached rows
+    wide = np.stack([rng.permutation(256)[:8] for _ in range(tokens)])  # one: non-temporal rows
+    bad = wide.copy()
+    bad[77, 2] = 256
+    weights = torch.softmax(torch.from_numpy(rng.normal(size=(tokens, 8))), dim=1).to(torch.bfloat16).to(device)
+    ptrs = model.layers[0].expert_ptrs
+    indices = torch.from_numpy(wide.astype(np.int64)).to(device)
+    out = torch.empty_like(x)
+    ws, eager = Workspace(device, tokens), Workspace(device, tokens)
+    print("[units] captured call", flush=True)
+    moe_experts(x, indices, weights, ptrs, out=out, workspace=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        moe_experts(x, indices, weights, ptrs, out=out, workspace=ws)
+    for routes, status in ((few, 0), (wide, 0), (bad, 1), (few, 0), (few, 0), (wide, 0)):
+        indices.copy_(torch.from_numpy(routes.astype(np.int64)))
+        out.fill_(7.0)
+        graph.replay()
+        want = moe_experts(x, indices, weights, ptrs, workspace=eager)
+        torch.cuda.synchronize()
+        assert ws.status() == status and eager.status() == status
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+        assert bool(want.any()) == (status == 0)
